@@ -1,0 +1,71 @@
+"""The int8-dot decode GEMV (qgemv_dot.hip) at the edges of its shapes: one row, rows fewer and
+more than the CUs, units that do not fill the lanes of a row, rows of q3_K / q6_K that start
+two bytes off a dword, weights that start 4 bytes off a 16-byte boundary, K above the range of
+one pass over x, and block scales that are not finite.
+
+Bar: 2e-6 relative Frobenius against fp64.  Block sums are exact in int32 and rounded to
+fp32 once; a lane then adds at most K / (16 * 32) + 6 fp32 terms per row (34 at K = 14336,
+each rounding at most 2^-24 of the running sum), 2e-6 in the worst case.
+"""
+import numpy as np
+import pytest
+
+import oracle
+import tier_amd
+from tier_amd import hip
+
+pytestmark = pytest.mark.gpu
+T = tier_amd
+# one shape per type that the dot kernel takes, chosen so that no other kernel does
+SMALL = [T.Q4_0, T.Q4_1, T.Q5_0, T.Q5_1, T.IQ4_NL, T.Q8_0]
+SUPER = [T.Q2_K, T.Q3_K, T.IQ4_XS, T.Q4_K, T.Q5_K, T.Q6_K]
+SHAPES = [(1, 256), (3, 512), (255, 1280), (257, 2304), (600, 5376), (40, 14336), (17, 18432)]
+ODD_K = [(5, 64), (33, 320), (300, 1088)]
+
+
+def _run(blocks, t, x, N, K, offset=0):
+    rb = T.q_row_bytes(t, K)
+    W = hip.DeviceBuffer(N * rb + offset)
+    W.upload(np.ascontiguousarray(blocks).view(np.uint8).ravel(), offset)
+    X, Y = hip.to_device(x), hip.DeviceBuffer(N * 4)
+    Y.fill_bytes(0x3f)
+    T.gemv_q(W.ptr + offset, t, rb, X.ptr, Y.ptr, N, K)
+    hip.synchronize()
+    return Y.download(np.float32, N)
+
+
+def _blocks(t, N, K, seed):
+    rng = np.random.default_rng(seed)
+    return oracle.random_blocks(rng, t, N * (K // oracle.block(t)[0]), moderate=True).reshape(N, -1), \
+        rng.standard_normal(K).astype(np.float32)
+
+
+@pytest.mark.parametrize("t,N,K", [(t, N, K) for t in SMALL + SUPER for N, K in SHAPES] +
+                         [(t, N, K) for t in SMALL for N, K in ODD_K],
+                         ids=lambda v: str(v))
+def test_dot_gemv_shapes(gpu, t, N, K):
+    blocks, x = _blocks(t, N, K, 7 * N + K + t)
+    want = oracle.gemv_f64(blocks, t, x, N, K)
+    for offset in (0, 4) if t not in (T.Q4_K, T.Q5_K) else (0,):  # those rows are 16-byte aligned by contract
+        y = _run(blocks, t, x, N, K, offset)
+        assert np.all(np.isfinite(y))
+        assert oracle.rel_fro(y, want) <= 2e-6, offset
+
+
+@pytest.mark.parametrize("t", [T.Q4_0, T.Q5_1, T.IQ4_XS, T.Q2_K, T.Q3_K, T.Q6_K])
+def test_dot_gemv_nonfinite_scale(gpu, t):
+    """An infinite or NaN block scale: the row takes gemv_q's own classes, the others are untouched."""
+    N, K = 40, 1280
+    blocks, x = _blocks(t, N, K, 3 + t)
+    bb = oracle.block(t)[1]
+    at = {T.Q4_0: 0, T.Q5_1: 0, T.IQ4_XS: 0, T.Q2_K: 80, T.Q3_K: 108, T.Q6_K: 208}[t]
+    b = blocks.reshape(N, -1, bb)
+    for row, bits in ((3, 0x7c00), (11, 0xfc00), (30, 0x7e00)):
+        b[row, 2, at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+    y = _run(blocks, t, x, N, K)
+    want = oracle.gemv_lanes(blocks, t, x, N, K)
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        assert np.array_equal(f(y), f(want))
+    ok = np.isfinite(want)
+    assert ok.sum() == N - 3
+    assert oracle.rel_fro(y[ok], oracle.gemv_f64(blocks, t, x, N, K)[ok]) <= 2e-6

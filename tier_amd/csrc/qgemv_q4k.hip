@@ -217,30 +217,17 @@ int launch(const void* W, size_t rb, const float* x, float* y, int N, int K, hip
 // with the weight ring in the remaining 39 KiB).
 constexpr int kQ4kMaxK = 28672;
 
-// Launch shapes by measurement (MI355X; 200 launches over rotated copies).  At
-// most one row tile per CU: one tile per workgroup, K in four parts (q8_0
-// 4096x4096: 5.7 against 8.0 us).  Many row tiles: eight waves per workgroup
-// (q5_K 13824x5120: 11.7 against 15.1 us; q8_0 14336x14336: 41.5 against 46.6 us).
+// Launch shapes by measurement (MI355X; 200 launches over rotated copies), for the shapes
+// that neither the whole-tile kernel nor the dot kernel takes (qgemv_dispatch).  Many row
+// tiles: eight waves per workgroup.
 int qgemv_q4k(const void* W, size_t rb, const float* x, float* y, int N, int K, hipStream_t s) {
   if (K > kQ4kMaxK) return set_error(TIERMM_UNSUPPORTED, "tiermm_qgemv: q4_K K=%d above %d", K, kQ4kMaxK);
   const int tiles = (N + 15) / 16;
-  // 257..639 row tiles (taller ones take the whole-tile kernel): two tiles x four K
-  // parts per workgroup (q4_K 5120x5120: 5.6 against 6.4 us; 10000x5120: 9.0 against
-  // 10.2; 4608x8192: 6.6 against 8.4)
-  if (K <= 5120) {
-    if (tiles <= 256) return launch<QT_Q4_K, 1, 4, 1, 3, 2, 5120>(W, rb, x, y, N, K, s);
-    return launch<QT_Q4_K, 2, 4, 1, 2, 1, 5120>(W, rb, x, y, N, K, s);
-  }
-  if (K <= 8192) {
-    if (tiles <= 256) return launch<QT_Q4_K, 2, 2, 2, 3, 2, 8192>(W, rb, x, y, N, K, s);
-    return launch<QT_Q4_K, 2, 4, 2, 2, 1, 8192>(W, rb, x, y, N, K, s);
-  }
+  // 257..639 row tiles: two tiles x four K parts per workgroup (4608x8192: 6.6 against 8.4 us)
+  if (K <= 8192) return launch<QT_Q4_K, 2, 4, 2, 2, 1, 8192>(W, rb, x, y, N, K, s);
   // K above 14336: eight waves (two tiles x four K parts), one super-block per stage
   if (K > 14336) return launch<QT_Q4_K, 2, 4, 1, 2, 4, 28672>(W, rb, x, y, N, K, s);
   if (tiles >= 640) return launch<QT_Q4_K, 4, 1, 4, 2, 4, 14336>(W, rb, x, y, N, K, s);  // 24.2 against 25.5 us
-  // up to one tile per CU: one tile, K in eight parts (4096x14336: 9.4-9.6 against 11.7 us;
-  // 1024x14336: 7.1 against 9.4 us)
-  if (tiles <= 256) return launch<QT_Q4_K, 1, 8, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);
   return launch<QT_Q4_K, 2, 4, 2, 2, 2, 14336>(W, rb, x, y, N, K, s);
 }
 
@@ -254,35 +241,19 @@ bool qgemv_mfma_fits(const void* W, int qtype, size_t rb, int K) {
 int qgemv_mfma(const void* W, int qtype, size_t rb, const float* x, float* y, int N, int K, hipStream_t s) {
   const int tiles = (N + 15) / 16;
   if (qtype == QT_Q5_K) {
-    if (K <= 5120) {
-      if (tiles <= 256) return launch<QT_Q5_K, 1, 4, 1, 3, 2, 5120>(W, rb, x, y, N, K, s);
-      if (tiles < 640) return launch<QT_Q5_K, 2, 4, 1, 2, 2, 5120>(W, rb, x, y, N, K, s);
-      return launch<QT_Q5_K, 4, 2, 2, 2, 2, 5120>(W, rb, x, y, N, K, s);
-    }
-    if (K <= 8192) {
-      if (tiles < 640) return launch<QT_Q5_K, 2, 2, 2, 3, 2, 8192>(W, rb, x, y, N, K, s);
-      return launch<QT_Q5_K, 4, 2, 2, 2, 2, 8192>(W, rb, x, y, N, K, s);
-    }
+    if (K <= 5120) return launch<QT_Q5_K, 1, 4, 1, 3, 2, 5120>(W, rb, x, y, N, K, s);  // below 64 row tiles
+    if (K <= 8192) return launch<QT_Q5_K, 2, 2, 2, 3, 2, 8192>(W, rb, x, y, N, K, s);  // 64..639
     if (K > 14336) return launch<QT_Q5_K, 2, 3, 1, 2, 5, 28672>(W, rb, x, y, N, K, s);  // six waves fit the ring
     if (tiles >= 640) return launch<QT_Q5_K, 4, 2, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);
-    if (tiles <= 256) return launch<QT_Q5_K, 1, 8, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);  // 4096x14336: 11.0 against 13.8 us
     return launch<QT_Q5_K, 2, 4, 2, 2, 2, 14336>(W, rb, x, y, N, K, s);
   }
   if (K <= 5120) {
-    // 2048x4096: 4.4 against 5.1 us with K in four parts
+    // at most one row tile per CU: one tile per workgroup, K in eight parts
     if (tiles <= 256) return launch<QT_Q8_0, 1, 8, 1, 2, 1, 5120>(W, rb, x, y, N, K, s);
-    if (tiles < 640) return launch<QT_Q8_0, 2, 2, 1, 3, 2, 5120>(W, rb, x, y, N, K, s);
-    return launch<QT_Q8_0, 4, 2, 2, 2, 2, 5120>(W, rb, x, y, N, K, s);
-  }
-  if (K <= 8192) {
-    if (tiles < 640) return launch<QT_Q8_0, 2, 2, 1, 3, 2, 8192>(W, rb, x, y, N, K, s);
-    return launch<QT_Q8_0, 4, 2, 1, 2, 2, 8192>(W, rb, x, y, N, K, s);
+    return launch<QT_Q8_0, 2, 2, 1, 3, 2, 5120>(W, rb, x, y, N, K, s);
   }
   if (K > 14336) return launch<QT_Q8_0, 1, 4, 1, 2, 7, 28672>(W, rb, x, y, N, K, s);  // four waves fit the ring
-  if (tiles >= 640) return launch<QT_Q8_0, 4, 2, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);
-  // 1024x14336: 9.3 against 16.7 us; 4096x14336: 14.5 against 18.9 us
-  if (tiles <= 256) return launch<QT_Q8_0, 1, 8, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);
-  return launch<QT_Q8_0, 2, 2, 2, 2, 4, 14336>(W, rb, x, y, N, K, s);
+  return launch<QT_Q8_0, 1, 8, 1, 2, 2, 14336>(W, rb, x, y, N, K, s);  // 4096x14336: 14.5 against 18.9 us
 }
 
 }  // namespace tiermm
