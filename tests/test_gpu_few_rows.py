@@ -1,0 +1,114 @@
+"""The few-row quantized GEMM (qgemm_skinny.hip) at the edges of its shapes: row counts around
+its 16-row tiles and its largest, widths that leave a partial tile, one unit of K and several,
+units cut short (K not a multiple of 256), rows that start in the middle of a dword, x and Y off
+a 16-byte boundary, beta, experts of different sizes and types in one call.
+
+Bars.  F32: 2^-20 against fp64 (x in 22 bits, the weights exact, at most K / 4 products in one
+fp32 sum).  x3-ref: 2^-20 against the fp64 product with the fp16 weight; and bit for bit on unit
+vectors, whose product is a column of the fp16 weight itself.  Errors are relative to the root of
+the summed squares of all products x_k w_k: the Frobenius norm that random signs give, and what the
+rounding errors scale with also where a call has so few outputs that theirs cancel (one, here).
+"""
+import numpy as np
+import pytest
+
+import oracle
+import tier_amd
+from helpers import activations, quantized_weight
+from tier_amd import hip
+
+pytestmark = pytest.mark.gpu
+BAR = 2.0 ** -20
+T = tier_amd
+TYPES = [T.Q4_K, T.Q5_K, T.Q6_K, T.Q8_0, T.Q5_0]
+SHAPES = [(1, 1, 256), (2, 300, 512), (15, 128, 1280), (16, 129, 768), (17, 1000, 2048), (32, 257, 2304),
+          (37, 130, 3328), (48, 640, 5120), (49, 64, 1024)]
+TAILS = [(2, 70, 32), (7, 129, 416), (16, 200, 1408), (33, 40, 5088)]  # q8_0 / q5_0
+
+
+def _weight(t, N, K, seed, out):
+    blocks = quantized_weight(t, N, K, seed)
+    w = oracle.dequant(blocks, t, K, out)
+    w = w if out == oracle.OUT_F32 else oracle.h2f_array(w)
+    return blocks, w.reshape(N, K).astype(np.float64)
+
+
+def _err(got, want, x, w):
+    scale = np.sqrt(((x.astype(np.float64) ** 2) @ (w ** 2).T).sum())
+    return np.linalg.norm(got.astype(np.float64) - want) / scale
+
+
+def _run(blocks, t, x, N, K, mode, y0=None, ldy=None, off=0):
+    """The product with x and Y `off` bytes into their buffers; y0 (M, ldy) given: beta = 1."""
+    M, ldy = x.shape[0], ldy or N
+    W, X, Y = hip.to_device(blocks), hip.DeviceBuffer(x.nbytes + off), hip.DeviceBuffer(M * ldy * 4 + off)
+    X.upload(x, off)
+    Y.upload(np.full(M * ldy, 7.5, np.float32) if y0 is None else y0, off)
+    T.qgemm(W.ptr, t, T.q_row_bytes(t, K), X.ptr + off, Y.ptr + off, M, N, K, ldy=ldy, mode=mode,
+            beta=0.0 if y0 is None else 1.0)
+    hip.synchronize()
+    return Y.download(np.float32, M * ldy, off).reshape(M, ldy)
+
+
+@pytest.mark.parametrize("mode", [T.MODE_F32, T.MODE_X3REF], ids=["f32", "x3ref"])
+@pytest.mark.parametrize("t,M,N,K", [(t, *s) for t in TYPES for s in SHAPES] +
+                         [(t, *s) for t in (T.Q8_0, T.Q5_0) for s in TAILS], ids=lambda v: str(v))
+def test_few_rows(gpu, t, M, N, K, mode):
+    blocks, w = _weight(t, N, K, M + N + K + t, oracle.OUT_F32 if mode == T.MODE_F32 else oracle.OUT_F16)
+    x = activations(M, K, seed=M + t)
+    want = x.astype(np.float64) @ w.T
+    assert _err(_run(blocks, t, x, N, K, mode), want, x, w) <= BAR
+    y0 = np.random.default_rng(M).standard_normal((M, N + 3)).astype(np.float32)
+    got = _run(blocks, t, x, N, K, mode, y0=y0, ldy=N + 3, off=4)
+    assert _err(got[:, :N], want + y0[:, :N], x, w) <= BAR + 2.0 ** -24 * np.linalg.norm(y0) / np.linalg.norm(want)
+    assert np.array_equal(got[:, N:], y0[:, N:])
+
+
+@pytest.mark.parametrize("t", TYPES)
+def test_few_rows_x3ref_weight_bits(gpu, t):
+    """Unit vectors: every product is one fp16 weight, exactly the dequant's bits."""
+    M, N, K = 16, 400, 768
+    blocks, w = _weight(t, N, K, 5 + t, oracle.OUT_F16)
+    cols = np.random.default_rng(t).choice(K, (12, M), replace=False)
+    for c in cols:
+        x = np.zeros((M, K), np.float32)
+        x[np.arange(M), c] = 1.0
+        assert np.array_equal(_run(blocks, t, x, N, K, T.MODE_X3REF).astype(np.float64), w[:, c].T)
+
+
+def test_few_rows_nonfinite_scale(gpu):
+    """A block scale that is not finite makes its weight row's outputs NaN and no others."""
+    M, N, K = 5, 40, 512
+    for t, at in ((T.Q4_K, 0), (T.Q6_K, 208), (T.Q8_0, 0)):
+        blocks, w = _weight(t, N, K, 9 + t, oracle.OUT_F32)
+        b = blocks.reshape(N, -1, oracle.block(t)[1]).copy()
+        for row, bits in ((3, 0x7c00), (11, 0x7e00)):
+            b[row, 1, at:at + 2] = np.array([bits], np.uint16).view(np.uint8)
+        x = activations(M, K, seed=t)
+        y = _run(b.reshape(N, -1), t, x, N, K, T.MODE_F32)
+        bad = np.isin(np.arange(N), (3, 11))
+        assert np.all(np.isnan(y[:, bad]))
+        assert oracle.rel_fro(y[:, ~bad], (x.astype(np.float64) @ w.T)[:, ~bad]) <= BAR
+
+
+@pytest.mark.parametrize("N,K", [(1408, 512), (130, 1408)])
+def test_few_rows_grouped(gpu, N, K):
+    """70 experts (more than one launch holds) of 0 to 40 rows and of alternating types, more tiles
+    than the CUs: every expert's rows equal its own product."""
+    E = 70
+    types = [T.Q8_0, T.Q5_0, T.Q8_0] if K % 256 else [T.Q4_K, T.Q5_0, T.Q6_K]
+    rng = np.random.default_rng(N)
+    sizes = rng.choice([0, 1, 2, 3, 16], E)
+    sizes[5] = 16 if K % 256 else 31
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    P = int(offs[-1])
+    x = activations(P, K, seed=N)
+    qts = [types[e % 3] for e in range(E)]
+    made = {t: _weight(t, N, K, 3 + t, oracle.OUT_F16) for t in set(types)}
+    bufs = {t: hip.to_device(made[t][0]) for t in made}
+    X, Y = hip.to_device(x), hip.DeviceBuffer(P * N * 4)
+    T.qgemm_grouped([bufs[t].ptr for t in qts], qts, [T.q_row_bytes(t, K) for t in qts], X.ptr, offs, Y.ptr, N, K)
+    hip.synchronize()
+    got = Y.download(np.float32, P * N).reshape(P, N)
+    want = np.concatenate([x[offs[e]:offs[e + 1]].astype(np.float64) @ made[qts[e]][1].T for e in range(E)])
+    assert oracle.rel_fro(got, want) <= BAR

@@ -999,6 +999,8 @@ QPlan q_plan(int qt, const int* rows, int n, int N, int K, int cus, bool split, 
   return best;
 }
 
+}  // namespace
+
 // CUs of the current device, or 256 (MI355X) where no device is visible (a size
 // query on a host without a GPU); no error is recorded for that case.
 int cus_or_default() {
@@ -1006,8 +1008,6 @@ int cus_or_default() {
   if (hipGetDevice(&dev) != hipSuccess) return 256;
   return device_cus(&cus) == TIERMM_OK && cus > 0 ? cus : 256;
 }
-
-}  // namespace
 
 // Bytes of split-K partial sums the fused GEMM of one M x N x K problem needs.
 size_t qgemm_fused_partials_bytes(int qtype, int M, int N, int K, bool f32) {
@@ -1022,6 +1022,21 @@ size_t qgemm_fused_partials_bytes(int qtype, int M, int N, int K, bool f32) {
 bool qgemm_fusable(int qtype, const int* rows, int n, int N, int K, bool split, bool f32) {
   if (f32 && n != 1) return false;
   return q_plan(qtype, rows, n, N, K, cus_or_default(), split && n == 1, f32).bn != 0;
+}
+
+// Y (beta)= the ks partial sums P + z * ps of rows x N, in split order.
+int qgemm_splitk_sum(const float* P, size_t ps, int ks, float* Y, int ldy, int rows, int N, float beta, hipStream_t s,
+                     const char* who) {
+  if (N % 4 == 0 && ldy % 4 == 0 && rows <= 65535 && ((uintptr_t)Y & 15) == 0 && ((uintptr_t)P & 15) == 0 &&
+      ps % 4 == 0) {
+    const dim3 grid((unsigned)((N / 4 + 255) / 256), (unsigned)rows);
+    qgemm_splitk_reduce4<<<grid, 256, 0, s>>>(P, ps, ks, Y, ldy, N, beta);
+  } else {
+    const size_t cnt = (size_t)rows * N;
+    qgemm_splitk_reduce<<<(unsigned)((cnt + 255) / 256), 256, 0, s>>>(P, ps, ks, Y, ldy, rows, N, beta);
+  }
+  TM_LAUNCH_CHECK(who);
+  return TIERMM_OK;
 }
 
 // Fused x3-ref GEMM over n groups (rows[g] rows of x from row0[g], qtype weight W[g]);
@@ -1064,17 +1079,8 @@ int qgemm_fused_groups(const void* const* W, int qtype, const int* row0, const i
     }
     if (st) return st;
     if (pl.ks > 1) {  // n == 1, kc == 1: rows row0[0].. of Y
-      float* y0 = Y + (size_t)row0[0] * ldy;
-      if (N % 4 == 0 && ldy % 4 == 0 && rows[0] <= 65535 && ((uintptr_t)y0 & 15) == 0 &&
-          ((uintptr_t)partials & 15) == 0 && a.ps % 4 == 0) {
-        const dim3 grid((unsigned)((N / 4 + 255) / 256), (unsigned)rows[0]);
-        qgemm_splitk_reduce4<<<grid, 256, 0, s>>>(partials, a.ps, pl.ks, y0, ldy, N, beta);
-      } else {
-        const size_t cnt = (size_t)rows[0] * N;
-        qgemm_splitk_reduce<<<(unsigned)((cnt + 255) / 256), 256, 0, s>>>(partials, a.ps, pl.ks, y0, ldy, rows[0], N,
-                                                                         beta);
-      }
-      TM_LAUNCH_CHECK(who);
+      st = qgemm_splitk_sum(partials, a.ps, pl.ks, Y + (size_t)row0[0] * ldy, ldy, rows[0], N, beta, s, who);
+      if (st) return st;
     }
   }
   return TIERMM_OK;

@@ -49,6 +49,14 @@ int qrow_exps(const void* W, int qtype, size_t rb, int N, int K, int32_t* wexp, 
 int f32_prep(const float* X, uint16_t* xhi, uint16_t* xlo, int32_t* xexp, int M, int K, const void* W, int qtype,
              size_t rb, int N, int32_t* wexp, hipStream_t s);
 int device_cus(int* cus);
+// the few-row kernel (qgemm_skinny.hip)
+bool qgemm_skinny_takes(int qt, int M, int N, int K, bool f32);
+size_t qgemm_skinny_ws_bytes(int qt, int M, int N, int K, bool f32, int cus);
+size_t qgemm_skinny_group_ws_bytes(int qt, const int* rows, int n, int N, int K);
+int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows, int n, size_t rb, const float* X,
+                 const uint16_t* xparts, size_t pstride, size_t kt, float* Y, int ldy, int N, int K, float beta, bool f32,
+                 void* ws, int cus, hipStream_t s, const char* who);
+int cus_or_default();
 
 namespace {
 
@@ -998,6 +1006,36 @@ bool grouped_fused(int qt, const int* qts, const int* offs, int n_experts, int N
   return !rows.empty() && qgemm_fusable(qt, rows.data(), (int)rows.size(), N, K, false);
 }
 
+// Few rows take the few-row kernel, unless TIERMM_QGEMM_TILE asks for a plan of the fused one.
+bool few_rows(int qt, int M, int N, int K, bool f32) {
+  return qgemm_skinny_takes(qt, M, N, K, f32) && !getenv("TIERMM_QGEMM_TILE");
+}
+// The routed experts of type qt (weights, first rows, row counts), and whether all have few rows.
+struct TypeGroups {
+  std::vector<const void*> W;
+  std::vector<int> row0, rows;
+  size_t rb = 0;
+  bool same_rb = true, few = true;
+};
+TypeGroups type_groups(int qt, const void* const* W_e, const int* qts, const size_t* rb_e, const int* offs, int n_experts,
+                       int N, int K) {
+  TypeGroups g;
+  g.few = K <= 4 * kAccChunkFrom && !getenv("TIERMM_QGEMM_TILE");  // (no K split over groups)
+  for (int e = 0; e < n_experts; ++e) {
+    const int Me = offs[e + 1] - offs[e];
+    if (Me == 0 || qts[e] != qt) continue;
+    if (rb_e) {
+      g.same_rb = g.same_rb && (!g.rb || rb_e[e] == g.rb);
+      g.rb = rb_e[e];
+      g.W.push_back(W_e[e]);
+    }
+    g.row0.push_back(offs[e]);
+    g.rows.push_back(Me);
+    g.few = g.few && qgemm_skinny_takes(qt, Me, N, K, false);
+  }
+  return g;
+}
+
 // The distinct weight types of the routed experts, each with whether grouped_fused takes it.
 std::vector<std::pair<int, bool>> routed_types(const int* qts, const int* offs, int n_experts, int N, int K) {
   std::vector<std::pair<int, bool>> t;
@@ -1457,6 +1495,8 @@ size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
     }
     return al256((size_t)N * kp * 2) + (size_t)3 * M * kp * sizeof(uint16_t);  // padded W16, x planes
   }
+  if (few_rows(qtype, M, N, K, mode == TIERMM_MODE_F32))
+    return qgemm_skinny_ws_bytes(qtype, M, N, K, mode == TIERMM_MODE_F32, cus_or_default());
   if (mode == TIERMM_MODE_F32) {
     if (qgemm_fusable(qtype, &M, 1, N, K, true, true))  // x's two-part split, both exponent rows; split-K partials
       return 2 * al256((size_t)M * K * 2) + al256((size_t)M * 4) + al256((size_t)N * 4) +
@@ -1489,6 +1529,14 @@ int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, 
   hipStream_t s = (hipStream_t)stream;
   if (K % BK) return qgemm_padded(W, qtype, rb, X, Y, M, N, K, ldy, mode, beta, w, s, who);
   const size_t mk = (size_t)M * K;
+  if (few_rows(qtype, M, N, K, mode == TIERMM_MODE_F32)) {
+    int cus = 0;
+    st = device_cus(&cus);
+    if (st) return st;
+    const int row0 = 0;
+    return qgemm_skinny(&W, qtype, &row0, &M, 1, rb, X, nullptr, 0, 0, Y, ldy, N, K, beta, mode == TIERMM_MODE_F32, w, cus,
+                        s, who);
+  }
   if (mode == TIERMM_MODE_F32 && qgemm_fusable(qtype, &M, 1, N, K, true, true)) {
     // the same semantics with W decoded inside the GEMM: no fp32 or fp16 copy of W
     // in memory; one pass over the weight's block scales for its row exponents first
@@ -1576,6 +1624,7 @@ int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, 
 
 size_t tiermm_qgemm_x3parts_ws_bytes(int qtype, int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
+  if (few_rows(qtype, M, N, K, false)) return qgemm_skinny_ws_bytes(qtype, M, N, K, false, cus_or_default());
   if (qgemm_fusable(qtype, &M, 1, N, K, true)) return qgemm_fused_partials_bytes(qtype, M, N, K);
   return (size_t)N * K * sizeof(uint16_t);  // the fp16 weight
 }
@@ -1600,6 +1649,14 @@ int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xp
   st = get_workspace(ws, ws_bytes, tiermm_qgemm_x3parts_ws_bytes(qtype, M, N, K), &w, who);
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
+  if (few_rows(qtype, M, N, K, false)) {  // the kernel that tiermm_qgemm takes on the unsplit x
+    int cus = 0;
+    st = device_cus(&cus);
+    if (st) return st;
+    const int row0 = 0;
+    return qgemm_skinny(&W, qtype, &row0, &M, 1, rb, nullptr, xparts, part_stride, tiled ? (size_t)M : 0, Y, ldy, N, K, beta,
+                        false, w, cus, s, who);
+  }
   if (qgemm_fusable(qtype, &M, 1, N, K, true)) {
     int cus = 0;
     st = device_cus(&cus);
@@ -1634,8 +1691,15 @@ size_t tiermm_qgemm_grouped_ws_bytes(const int* qtype_e, const int* expert_offse
   // experts that are not decoded inside the GEMM)
   const size_t P = n_experts > 0 ? (size_t)expert_offsets[n_experts] : 0;
   const auto types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
-  bool staged = false;
-  for (auto& t : types) staged = staged || !t.second;
+  bool staged = false, all_few = !types.empty();
+  size_t few = 0;  // the fragments of the types whose experts all have few rows
+  for (auto& t : types) {
+    staged = staged || !t.second;
+    const auto g = type_groups(t.first, nullptr, qtype_e, nullptr, expert_offsets, n_experts, N, K);
+    all_few = all_few && t.second && g.few;
+    if (g.few) few = std::max(few, qgemm_skinny_group_ws_bytes(t.first, g.rows.data(), (int)g.rows.size(), N, K));
+  }
+  if (all_few) return few;
   const int chunk = staged && n_experts > 0 ? big_group_chunk(expert_offsets, n_experts, N, K) : 0;
   if (chunk) return al256(3 * P * K * sizeof(uint16_t)) + chunk * al256((size_t)N * K * sizeof(uint16_t));
   return al256(3 * P * K * sizeof(uint16_t)) + (staged ? (size_t)N * K * sizeof(uint16_t) : 0);
@@ -1674,6 +1738,30 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
       if (st) return st;
     }
     return TIERMM_OK;
+  }
+  int cus = 0;
+  st = device_cus(&cus);
+  if (st) return st;
+  // Experts with few rows each (a batched decode step): the few-row kernel, one launch per type,
+  // where every routed type's experts are such
+  {
+    const auto types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
+    std::vector<TypeGroups> gs;
+    bool few = !types.empty();
+    for (auto& t : types) {
+      gs.push_back(type_groups(t.first, W_e, qtype_e, rb_e, expert_offsets, n_experts, N, K));
+      few = few && t.second && gs.back().few;
+    }
+    if (few) {
+      for (size_t i = 0; i < types.size(); ++i) {
+        const auto& g = gs[i];
+        if (!g.same_rb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
+        st = qgemm_skinny(g.W.data(), types[i].first, g.row0.data(), g.rows.data(), (int)g.rows.size(), g.rb, X_sorted,
+                          nullptr, 0, 0, Y_sorted, N, N, K, 0.f, false, w, cus, s, who);
+        if (st) return st;
+      }
+      return TIERMM_OK;
+    }
   }
   // x3-ref: split every routed row once; each expert multiplies its slice of the planes
   const size_t P = (size_t)expert_offsets[n_experts], pk = P * K;
@@ -1738,26 +1826,13 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
     }
     return TIERMM_OK;
   }
-  int cus = 0;
-  st = device_cus(&cus);
-  if (st) return st;
   // experts of each fused type: one launch (per 64 experts) whose workgroups cover every
   // expert's tiles
   for (auto& t : types) {
     if (!t.second) continue;
-    std::vector<const void*> gw;
-    std::vector<int> g0, gr;
-    size_t grb = 0;
-    for (int e = 0; e < n_experts; ++e) {
-      const int o = expert_offsets[e], Me = expert_offsets[e + 1] - o;
-      if (Me == 0 || qtype_e[e] != t.first) continue;
-      if (grb && rb_e[e] != grb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
-      grb = rb_e[e];
-      gw.push_back(W_e[e]);
-      g0.push_back(o);
-      gr.push_back(Me);
-    }
-    st = qgemm_fused_groups(gw.data(), t.first, g0.data(), gr.data(), (int)gw.size(), grb, parts, pk,
+    const auto g = type_groups(t.first, W_e, qtype_e, rb_e, expert_offsets, n_experts, N, K);
+    if (!g.same_rb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
+    st = qgemm_fused_groups(g.W.data(), t.first, g.row0.data(), g.rows.data(), (int)g.rows.size(), g.rb, parts, pk,
                             tiled ? P : 0, Y_sorted, N, N, K, 0.f, cus, s, who, nullptr);
     if (st) return st;
   }
