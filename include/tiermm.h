@@ -258,7 +258,9 @@ size_t tiermm_sgemm_ws_bytes(int opA, int m, int n, int k);
  * Frobenius error <= 2^-20 against fp64(deq(W) * X).  qtype: the GPU types of
  * tiermm_dequant.  The workspace (tiermm_qgemm_ws_bytes) holds the x parts and,
  * for q8_0 / q4_K / q5_K / q6_K / q5_0 (decoded inside the GEMM), the split-K partial
- * sums, or for the other types the fp16 weight; the environment variable
+ * sums, or for the other types the fp16 weight; a call of few rows whose workspace
+ * (sized for another M) has no room for the few-row kernel's sums takes the tiled
+ * kernel.  The environment variable
  * TIERMM_QGEMM_TILE="BN,KS[,KC]" overrides the fused kernel's tile width, split count
  * and accumulation chunks (read at each call, and by the size query; ignored when
  * invalid for the shape). */

@@ -22,7 +22,7 @@ BAR = 2.0 ** -20
 T = tier_amd
 TYPES = [T.Q4_K, T.Q5_K, T.Q6_K, T.Q8_0, T.Q5_0]
 SHAPES = [(1, 1, 256), (2, 300, 512), (15, 128, 1280), (16, 129, 768), (17, 1000, 2048), (32, 257, 2304),
-          (37, 130, 3328), (48, 640, 5120), (49, 64, 1024)]
+          (37, 130, 3328), (48, 640, 5120), (49, 64, 1024), (4, 65, 768), (5, 200, 512), (8, 300, 1280), (9, 70, 512)]
 TAILS = [(2, 70, 32), (7, 129, 416), (16, 200, 1408), (33, 40, 5088)]  # q8_0 / q5_0
 
 
@@ -112,3 +112,18 @@ def test_few_rows_grouped(gpu, N, K):
     got = Y.download(np.float32, P * N).reshape(P, N)
     want = np.concatenate([x[offs[e]:offs[e + 1]].astype(np.float64) @ made[qts[e]][1].T for e in range(E)])
     assert oracle.rel_fro(got, want) <= BAR
+
+
+@pytest.mark.parametrize("mode", [T.MODE_F32, T.MODE_X3REF], ids=["f32", "x3ref"])
+@pytest.mark.parametrize("t,M,N,K", [(T.Q4_K, 16, 1024, 4096), (T.Q8_0, 3, 300, 1408)])
+def test_few_rows_in_a_workspace_of_the_general_path(gpu, t, M, N, K, mode):
+    """A workspace that an M of the general path was sized for: too small for the split sums of the
+    few-row kernel, which then leaves the call to the general path."""
+    blocks, w = _weight(t, N, K, 3, oracle.OUT_F32 if mode == T.MODE_F32 else oracle.OUT_F16)
+    x = activations(M, K, seed=4)
+    W, X, Y = hip.to_device(blocks), hip.to_device(x), hip.DeviceBuffer(M * N * 4)
+    for size in (T.qgemm_ws_bytes(t, 64, N, K, mode), T.qgemm_ws_bytes(t, M, N, K, mode)):
+        ws = hip.DeviceBuffer(size)
+        T.qgemm(W.ptr, t, T.q_row_bytes(t, K), X.ptr, Y.ptr, M, N, K, mode=mode, ws=ws.ptr, ws_bytes=size)
+        hip.synchronize()
+        assert _err(Y.download(np.float32, M * N).reshape(M, N), x.astype(np.float64) @ w.T, x, w) <= BAR

@@ -56,6 +56,18 @@ int hip_fail(int hip_err, const char* what) {
   return -hip_err;
 }
 
+bool workspace_holds(void* ws, size_t ws_bytes, size_t need, void* stream) {
+  if (ws) return ws_bytes >= need;
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return true;  // get_workspace reports it
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    if ((int)g_pools.size() > dev && g_pools[dev].bytes >= need) return true;
+  }
+  hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing((hipStream_t)stream, &c) != hipSuccess || c == hipStreamCaptureStatusNone;
+}
+
 int get_workspace(void* ws, size_t ws_bytes, size_t need, void** out, const char* who) {
   if (need == 0) {
     *out = ws;

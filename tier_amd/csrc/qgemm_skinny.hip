@@ -849,6 +849,11 @@ size_t qgemm_skinny_group_ws_bytes(int qt, const int* rows, int n, int N, int K)
   return sk_ws(qt, mtot, r, N, K, false, 1).total;
 }
 
+// An upper bound of the same over every routing of P rows to n experts.
+size_t qgemm_skinny_routed_ws_bytes(size_t P, int n, int K) {
+  return sk_ws(QT_Q4_K, std::min(P, (size_t)n + P / 16), P, 0, K, false, 1).total;
+}
+
 int qgemm_splitk_sum(const float* P, size_t ps, int ks, float* Y, int ldy, int rows, int N, float beta, hipStream_t s,
                      const char* who);
 

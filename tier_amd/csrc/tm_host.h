@@ -33,6 +33,9 @@ int hip_fail(int hip_err, const char* what);
 // Workspace: caller-provided (ws != nullptr) or the per-device pool.
 // Returns TIERMM_OK and sets *out, or an error status.
 int get_workspace(void* ws, size_t ws_bytes, size_t need, void** out, const char* who);
+// Whether get_workspace would give `need` bytes: a caller's workspace of that size, or a pool that
+// has them or may grow (not while `stream` is being captured).
+bool workspace_holds(void* ws, size_t ws_bytes, size_t need, void* stream);
 
 int quantize_rows(int qtype, const float* x, void* out, size_t rows, int cols, int nthreads);
 

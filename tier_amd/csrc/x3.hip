@@ -53,6 +53,7 @@ int device_cus(int* cus);
 bool qgemm_skinny_takes(int qt, int M, int N, int K, bool f32);
 size_t qgemm_skinny_ws_bytes(int qt, int M, int N, int K, bool f32, int cus);
 size_t qgemm_skinny_group_ws_bytes(int qt, const int* rows, int n, int N, int K);
+size_t qgemm_skinny_routed_ws_bytes(size_t P, int n, int K);
 int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows, int n, size_t rb, const float* X,
                  const uint16_t* xparts, size_t pstride, size_t kt, float* Y, int ldy, int N, int K, float beta, bool f32,
                  void* ws, int cus, hipStream_t s, const char* who);
@@ -1010,6 +1011,12 @@ bool grouped_fused(int qt, const int* qts, const int* offs, int n_experts, int N
 bool few_rows(int qt, int M, int N, int K, bool f32) {
   return qgemm_skinny_takes(qt, M, N, K, f32) && !getenv("TIERMM_QGEMM_TILE");
 }
+// What the few-row kernel needs of a product that it takes (0: it does not take it).  Its need
+// falls and rises with M otherwise than the general path's, so the size queries return the larger of
+// the two, and a workspace (sized for another M, say) that holds only the general path's runs that.
+size_t few_rows_ws_bytes(int qt, int M, int N, int K, bool f32) {
+  return few_rows(qt, M, N, K, f32) ? qgemm_skinny_ws_bytes(qt, M, N, K, f32, cus_or_default()) : 0;
+}
 // The routed experts of type qt (weights, first rows, row counts), and whether all have few rows.
 struct TypeGroups {
   std::vector<const void*> W;
@@ -1485,7 +1492,7 @@ int tiermm_sgemm(int opA, int m, int n, int k, const float* A, int lda, const fl
   return launch_x3<128, 128, X3_2X2>(a, s, who);
 }
 
-size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
+static size_t qgemm_general_ws_bytes(int qtype, int M, int N, int K, int mode) {
   if (K % BK) {  // dense rows of an odd length: W and x padded to rows of Kp
     const size_t kp = (size_t)pad32(K);
     if (mode == TIERMM_MODE_F32) {  // a chunk of padded fp32 W rows, padded fp32 x, their two-part splits
@@ -1495,8 +1502,6 @@ size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
     }
     return al256((size_t)N * kp * 2) + (size_t)3 * M * kp * sizeof(uint16_t);  // padded W16, x planes
   }
-  if (few_rows(qtype, M, N, K, mode == TIERMM_MODE_F32))
-    return qgemm_skinny_ws_bytes(qtype, M, N, K, mode == TIERMM_MODE_F32, cus_or_default());
   if (mode == TIERMM_MODE_F32) {
     if (qgemm_fusable(qtype, &M, 1, N, K, true, true))  // x's two-part split, both exponent rows; split-K partials
       return 2 * al256((size_t)M * K * 2) + al256((size_t)M * 4) + al256((size_t)N * 4) +
@@ -1511,6 +1516,10 @@ size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
     return al256(parts) + qgemm_fused_partials_bytes(qtype, M, N, K);  // W decoded inside the GEMM; split-K partials
   return (size_t)N * K * sizeof(uint16_t) + parts;                   // W16 staged in the workspace
 }
+size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
+  const size_t few = K % BK ? 0 : few_rows_ws_bytes(qtype, M, N, K, mode == TIERMM_MODE_F32);
+  return std::max(few, qgemm_general_ws_bytes(qtype, M, N, K, mode));
+}
 
 int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, int M, int N, int K, int ldy,
                  int mode, float beta, void* ws, size_t ws_bytes, tiermm_stream_t stream) {
@@ -1524,12 +1533,14 @@ int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, 
   if (M == 0 || N == 0) return TIERMM_OK;
   if (!X || !Y) return set_error(TIERMM_EINVAL, "%s: null buffer", who);
   void* w = nullptr;
-  st = get_workspace(ws, ws_bytes, tiermm_qgemm_ws_bytes(qtype, M, N, K, mode), &w, who);
+  const size_t few = K % BK ? 0 : few_rows_ws_bytes(qtype, M, N, K, mode == TIERMM_MODE_F32);
+  const bool take_few = few && workspace_holds(ws, ws_bytes, few, stream);
+  st = get_workspace(ws, ws_bytes, take_few ? few : qgemm_general_ws_bytes(qtype, M, N, K, mode), &w, who);
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
   if (K % BK) return qgemm_padded(W, qtype, rb, X, Y, M, N, K, ldy, mode, beta, w, s, who);
   const size_t mk = (size_t)M * K;
-  if (few_rows(qtype, M, N, K, mode == TIERMM_MODE_F32)) {
+  if (take_few) {
     int cus = 0;
     st = device_cus(&cus);
     if (st) return st;
@@ -1622,11 +1633,13 @@ int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, 
   return launch_x3_big<X3_REF>(a, s, who);
 }
 
-size_t tiermm_qgemm_x3parts_ws_bytes(int qtype, int M, int N, int K) {
-  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
-  if (few_rows(qtype, M, N, K, false)) return qgemm_skinny_ws_bytes(qtype, M, N, K, false, cus_or_default());
+static size_t x3parts_general_ws_bytes(int qtype, int M, int N, int K) {
   if (qgemm_fusable(qtype, &M, 1, N, K, true)) return qgemm_fused_partials_bytes(qtype, M, N, K);
   return (size_t)N * K * sizeof(uint16_t);  // the fp16 weight
+}
+size_t tiermm_qgemm_x3parts_ws_bytes(int qtype, int M, int N, int K) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
+  return std::max(few_rows_ws_bytes(qtype, M, N, K, false), x3parts_general_ws_bytes(qtype, M, N, K));
 }
 
 int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xparts, size_t part_stride,
@@ -1646,10 +1659,12 @@ int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xp
     return set_error(TIERMM_EINVAL, "%s: x planes must be 16-byte aligned, part_stride >= M*K and a multiple of 8",
                      who);
   void* w = nullptr;
-  st = get_workspace(ws, ws_bytes, tiermm_qgemm_x3parts_ws_bytes(qtype, M, N, K), &w, who);
+  const size_t few = few_rows_ws_bytes(qtype, M, N, K, false);
+  const bool take_few = few && workspace_holds(ws, ws_bytes, few, stream);
+  st = get_workspace(ws, ws_bytes, take_few ? few : x3parts_general_ws_bytes(qtype, M, N, K), &w, who);
   if (st) return st;
   hipStream_t s = (hipStream_t)stream;
-  if (few_rows(qtype, M, N, K, false)) {  // the kernel that tiermm_qgemm takes on the unsplit x
+  if (take_few) {  // the kernel that tiermm_qgemm takes on the unsplit x
     int cus = 0;
     st = device_cus(&cus);
     if (st) return st;
@@ -1676,13 +1691,13 @@ int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xp
   return launch_x3_big<X3_REF>(a, s, who);
 }
 
-size_t tiermm_qgemm_grouped_ws_bytes(const int* qtype_e, const int* expert_offsets, int n_experts, int N, int K,
-                                     int mode) {
+static size_t grouped_general_ws_bytes(const int* qtype_e, const int* expert_offsets, int n_experts, int N, int K,
+                                       int mode) {
   size_t need = 0;
   if (mode == TIERMM_MODE_F32) {  // expert by expert through tiermm_qgemm
     for (int e = 0; e < n_experts; ++e) {
       const int Me = expert_offsets[e + 1] - expert_offsets[e];
-      if (Me > 0) need = std::max(need, tiermm_qgemm_ws_bytes(qtype_e[e], Me, N, K, mode));
+      if (Me > 0) need = std::max(need, qgemm_general_ws_bytes(qtype_e[e], Me, N, K, mode));
     }
     return need;
   }
@@ -1690,19 +1705,33 @@ size_t tiermm_qgemm_grouped_ws_bytes(const int* qtype_e, const int* expert_offse
   // chunk of experts (grouped 256x320 launch) or of one expert at a time (the
   // experts that are not decoded inside the GEMM)
   const size_t P = n_experts > 0 ? (size_t)expert_offsets[n_experts] : 0;
-  const auto types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
-  bool staged = false, all_few = !types.empty();
-  size_t few = 0;  // the fragments of the types whose experts all have few rows
-  for (auto& t : types) {
-    staged = staged || !t.second;
-    const auto g = type_groups(t.first, nullptr, qtype_e, nullptr, expert_offsets, n_experts, N, K);
-    all_few = all_few && t.second && g.few;
-    if (g.few) few = std::max(few, qgemm_skinny_group_ws_bytes(t.first, g.rows.data(), (int)g.rows.size(), N, K));
-  }
-  if (all_few) return few;
+  bool staged = false;
+  for (auto& t : routed_types(qtype_e, expert_offsets, n_experts, N, K)) staged = staged || !t.second;
   const int chunk = staged && n_experts > 0 ? big_group_chunk(expert_offsets, n_experts, N, K) : 0;
   if (chunk) return al256(3 * P * K * sizeof(uint16_t)) + chunk * al256((size_t)N * K * sizeof(uint16_t));
   return al256(3 * P * K * sizeof(uint16_t)) + (staged ? (size_t)N * K * sizeof(uint16_t) : 0);
+}
+// The few-row kernel's need of a routed batch (F32: of its experts, one after another).  The x-ref
+// bound holds for every routing of as many rows, as the general path's size does: a program may
+// size its workspace once and route anew.
+static size_t grouped_few_ws_bytes(const int* qtype_e, const int* expert_offsets, int n_experts, int N, int K, int mode) {
+  size_t need = 0;
+  if (mode == TIERMM_MODE_F32) {
+    for (int e = 0; e < n_experts; ++e)
+      need = std::max(need, K % BK ? 0 : few_rows_ws_bytes(qtype_e[e], expert_offsets[e + 1] - expert_offsets[e], N, K, true));
+    return need;
+  }
+  const size_t P = n_experts > 0 ? (size_t)expert_offsets[n_experts] : 0;
+  if (K % BK || K > 4 * kAccChunkFrom) return 0;
+  for (int e = 0; e < n_experts && !need; ++e)  // 48: more rows than the kernel takes of any expert
+    if (qgemm_skinny_takes(qtype_e[e], 1, N, K, false) && P <= (size_t)n_experts * 48)
+      need = qgemm_skinny_routed_ws_bytes(P, n_experts, K);
+  return need;
+}
+size_t tiermm_qgemm_grouped_ws_bytes(const int* qtype_e, const int* expert_offsets, int n_experts, int N, int K,
+                                     int mode) {
+  return std::max(grouped_general_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode),
+                  grouped_few_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode));
 }
 
 int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_t* rb_e, const float* X_sorted,
@@ -1724,7 +1753,28 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
   }
   if (n_experts == 0 || expert_offsets[n_experts] == 0 || N == 0) return TIERMM_OK;
   if (!X_sorted || !Y_sorted) return set_error(TIERMM_EINVAL, "%s: null buffer", who);
-  const size_t wsb = tiermm_qgemm_grouped_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode);
+  // Experts with few rows each (a batched decode step): the few-row kernel, one launch per type,
+  // where every routed type's experts are such
+  std::vector<std::pair<int, bool>> types;
+  std::vector<TypeGroups> gs;
+  size_t few = 0;
+  if (mode == TIERMM_MODE_F32) {
+    few = grouped_few_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode);
+    few = std::max(few, grouped_general_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode));
+  } else {
+    types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
+    for (auto& t : types) {
+      gs.push_back(type_groups(t.first, W_e, qtype_e, rb_e, expert_offsets, n_experts, N, K));
+      const auto& g = gs.back();
+      if (!t.second || !g.few) {
+        few = 0;
+        break;
+      }
+      few = std::max(few, qgemm_skinny_group_ws_bytes(t.first, g.rows.data(), (int)g.rows.size(), N, K));
+    }
+  }
+  const bool take_few = few && workspace_holds(ws, ws_bytes, few, stream);
+  const size_t wsb = take_few ? few : grouped_general_ws_bytes(qtype_e, expert_offsets, n_experts, N, K, mode);
   void* w = nullptr;
   st = get_workspace(ws, ws_bytes, wsb, &w, who);
   if (st) return st;
@@ -1742,26 +1792,15 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
   int cus = 0;
   st = device_cus(&cus);
   if (st) return st;
-  // Experts with few rows each (a batched decode step): the few-row kernel, one launch per type,
-  // where every routed type's experts are such
-  {
-    const auto types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
-    std::vector<TypeGroups> gs;
-    bool few = !types.empty();
-    for (auto& t : types) {
-      gs.push_back(type_groups(t.first, W_e, qtype_e, rb_e, expert_offsets, n_experts, N, K));
-      few = few && t.second && gs.back().few;
+  if (take_few) {
+    for (size_t i = 0; i < types.size(); ++i) {
+      const auto& g = gs[i];
+      if (!g.same_rb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
+      st = qgemm_skinny(g.W.data(), types[i].first, g.row0.data(), g.rows.data(), (int)g.rows.size(), g.rb, X_sorted,
+                        nullptr, 0, 0, Y_sorted, N, N, K, 0.f, false, w, cus, s, who);
+      if (st) return st;
     }
-    if (few) {
-      for (size_t i = 0; i < types.size(); ++i) {
-        const auto& g = gs[i];
-        if (!g.same_rb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
-        st = qgemm_skinny(g.W.data(), types[i].first, g.row0.data(), g.rows.data(), (int)g.rows.size(), g.rb, X_sorted,
-                          nullptr, 0, 0, Y_sorted, N, N, K, 0.f, false, w, cus, s, who);
-        if (st) return st;
-      }
-      return TIERMM_OK;
-    }
+    return TIERMM_OK;
   }
   // x3-ref: split every routed row once; each expert multiplies its slice of the planes
   const size_t P = (size_t)expert_offsets[n_experts], pk = P * K;
@@ -1772,7 +1811,6 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
   // 64 q4_K experts of ~512 rows, N = 1408, K = 2048: the MoE line 2.72 ms against
   // 2.86 ms).  Otherwise, where the experts' 256-row tiles fill the chip, every expert
   // goes through fp16 staging and the grouped big-tile launch.
-  const auto types = routed_types(qtype_e, expert_offsets, n_experts, N, K);
   bool all_fused = !types.empty();
   for (auto& t : types) all_fused = all_fused && t.second;
   const int chunk = all_fused ? 0 : big_group_chunk(expert_offsets, n_experts, N, K);
