@@ -41,6 +41,13 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 constexpr int SK_G = 64;          // groups per launch
 constexpr int SK_MT = 3;          // 16-row tiles of x, at most
 constexpr int SK_WR = 2;          // 16-row W tiles of a wave
+// Up to sk_pack rows, the parts of x share one MFMA tile: row m of part p at tile row m + p sk_pack
+// (x-ref three parts of 4 rows, F32 two of 8).  One product then does the work of three (two), x takes
+// a third (half) of the loads and LDS, and that room holds a third unit of weights in flight and the
+// meeting apart from the ring, so the loads no longer stop between two items.
+// Measured, us a call: 8 tokens, top 8 of 64 experts, hidden 2048, ffn 1408 (both products and the
+// combine) 127 -> 108, 1 token 44.7 -> 41.9; F32 q4_K 14336x5120 M = 8 27.1 -> 26.2.
+constexpr int sk_pack(bool f32) { return f32 ? 8 : 4; }
 // Row waves of a workgroup, each for four K quarters, by the row tiles of x
 constexpr int sk_rw(int mt) { return mt == 1 ? 2 : 4; }
 constexpr int sk_bn(int mt) { return 16 * SK_WR * sk_rw(mt); }
@@ -67,20 +74,21 @@ struct SkArgs {
 // s = 4 kh + 2 t + u.  (A lane's weights are then 16 consecutive elements of two
 // neighbouring 32-element blocks.)  PERM: the 8 halfs in the order 0 2 1 3 4 6 5 7, in
 // which the F32 decoders pair nibbles.
-template <int NP, bool PERM>
+template <int NP, bool PERM, bool PACK>
 __device__ __forceinline__ void put_frag(uint16_t* X, size_t mtot, size_t tile, int m, int k,
                                          const uint16_t (&h)[NP][8]) {
   const int r = k & 127, kg = 2 * (r >> 6) + ((r >> 4) & 1);
   const int s = 4 * ((k >> 7) & 1) + 2 * ((r >> 5) & 1) + ((r >> 3) & 1);
 #pragma unroll
   for (int p = 0; p < NP; ++p) {
-    const size_t f = ((size_t)((k >> 8) * 8 + s) * NP + p) * mtot + tile;
+    const size_t f = ((size_t)((k >> 8) * 8 + s) * (PACK ? 1 : NP) + (PACK ? 0 : p)) * mtot + tile;
+    const int row = PACK ? m + p * sk_pack(NP == 2) : m;
     const uint16_t(&v)[8] = h[p];
     const u32x4 o = PERM ? u32x4{v[0] | (uint32_t)v[2] << 16, v[1] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[6] << 16,
                                  v[5] | (uint32_t)v[7] << 16}
                          : u32x4{v[0] | (uint32_t)v[1] << 16, v[2] | (uint32_t)v[3] << 16, v[4] | (uint32_t)v[5] << 16,
                                  v[6] | (uint32_t)v[7] << 16};
-    *(u32x4*)(X + f * 512 + (16 * kg + m) * 8) = o;
+    *(u32x4*)(X + f * 512 + (16 * kg + row) * 8) = o;
   }
 }
 __device__ __forceinline__ void load8(const float* x, bool al, float (&v)[8]) {
@@ -108,6 +116,7 @@ __device__ __forceinline__ int row_place(const SkArgs& p, int i, size_t& tile, i
 
 // x-ref: the three fp16 parts (split3_fp_k, tier.cpp:869-870); one row per block.  K past the
 // row is zero up to a whole unit.
+template <bool PACK>
 __global__ __launch_bounds__(256) void sk_split3(const float* __restrict__ x, const SkArgs p,
                                                  uint16_t* __restrict__ X) {
   const int K = p.K, kp = (K + SK_UNIT - 1) / SK_UNIT * SK_UNIT;
@@ -127,11 +136,12 @@ __global__ __launch_bounds__(256) void sk_split3(const float* __restrict__ x, co
       h[1][e] = f2h(r1);
       h[2][e] = f2h(r1 - h2f(h[1][e]));
     }
-    put_frag<3, false>(X, p.mtot, tile, m, k, h);
+    put_frag<3, false, PACK>(X, p.mtot, tile, m, k, h);
   }
 }
 // The same fragments from parts that are split already (planes part_stride apart; kt > 0:
 // K-tiled over kt rows).
+template <bool PACK>
 __global__ __launch_bounds__(256) void sk_relayout3(const uint16_t* __restrict__ parts, size_t stride, size_t kt,
                                                     const SkArgs p, uint16_t* __restrict__ X) {
   const int K = p.K, kp = (K + SK_UNIT - 1) / SK_UNIT * SK_UNIT;
@@ -147,7 +157,7 @@ __global__ __launch_bounds__(256) void sk_relayout3(const uint16_t* __restrict__
 #pragma unroll
       for (int e = 0; e < 8; ++e) h[q][e] = (uint16_t)(w[e >> 1] >> (16 * (e & 1)));
     }
-    put_frag<3, false>(X, p.mtot, tile, m, k, h);
+    put_frag<3, false, PACK>(X, p.mtot, tile, m, k, h);
   }
 }
 
@@ -155,6 +165,7 @@ __global__ __launch_bounds__(256) void sk_relayout3(const uint16_t* __restrict__
 // sub-block sums S_b = sum of x * 2^e over the 32 elements of sub-block b, over 32, in two
 // fp16 parts: lane (m, kg) of the unit's sum fragment holds the hi parts of sub-blocks
 // 4 kg .. 4 kg + 3, then their lo parts, for kg < 2, and zeros beyond.
+template <bool PACK>
 __global__ __launch_bounds__(256) void sk_split2(const float* __restrict__ x, const SkArgs p, uint16_t* __restrict__ X,
                                                  uint16_t* __restrict__ S, int32_t* __restrict__ xexp) {
   __shared__ float red[4];
@@ -187,7 +198,7 @@ __global__ __launch_bounds__(256) void sk_split2(const float* __restrict__ x, co
       h[1][e] = f2h(f - h2f(h[0][e]));
       sum += f;
     }
-    put_frag<2, true>(X, p.mtot, tile, m, k, h);
+    put_frag<2, true, PACK>(X, p.mtot, tile, m, k, h);
     if (S) {  // four neighbouring lanes hold a sub-block
       sum += __shfl_xor(sum, 1, 64);
       sum += __shfl_xor(sum, 2, 64);
@@ -200,6 +211,9 @@ __global__ __launch_bounds__(256) void sk_split2(const float* __restrict__ x, co
         f[(16 * (b >> 2) + m) * 8 + 4 + (b & 3)] = s1;
       }
       if ((k & 255) == 16 || (k & 255) == 24) *(u32x4*)(f + (16 * ((k & 255) >> 3) + m) * 8) = u32x4{0, 0, 0, 0};
+      // the sums count once, with the hi parts
+      if (PACK && (k & 255) >= 32 && (k & 255) < 64)
+        *(u32x4*)(f + (16 * (((k & 255) - 32) >> 3) + m + sk_pack(true)) * 8) = u32x4{0, 0, 0, 0};
     }
   }
 }
@@ -465,10 +479,10 @@ struct Sk<QT_Q5_0> {
 
 // ---------------------------------------------------------------------- kernel
 constexpr int SK_LDS = 160 * 1024;
-template <int QT, bool F32, int MT>
+template <int QT, bool F32, int MT, bool PACK = false>
 struct SkLayout {
   using D = Sk<QT>;
-  static constexpr int NP = F32 ? 2 : 3;
+  static constexpr int NP = PACK ? 1 : F32 ? 2 : 3;  // x fragments of a step and tile
   static constexpr int RW = sk_rw(MT), WV = 4 * RW, BN = sk_bn(MT);
   static constexpr bool MINS = F32 && D::MINS;
   static constexpr int FR = (8 * NP + (MINS ? 1 : 0)) * MT;        // x fragments (KiB) of a unit
@@ -503,10 +517,10 @@ __device__ __forceinline__ void vm_wait_n(int n) {
   }
 }
 
-template <int QT, bool F32, int MT>
+template <int QT, bool F32, int MT, bool PACK>
 __global__ __launch_bounds__(256 * sk_rw(MT))
     __attribute__((amdgpu_waves_per_eu(4, 8))) void qgemm_skinny(const SkArgs p) {
-  using L = SkLayout<QT, F32, MT>;
+  using L = SkLayout<QT, F32, MT, PACK>;
   using D = Sk<QT>;
   constexpr int NP = L::NP, WR = SK_WR, PL = F32 ? D::PLANES : 1, CH = D::CH, ST = L::ST;
   extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -727,9 +741,17 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
     __syncthreads();
     for (int ij = quarter; ij < WR * MT; ij += 4) {
       const int i = ij / MT, j = ij % MT, col = it.n0 + (rw * WR + i) * 16 + n;
-      float4v v = red[(rw * WR * MT + ij) * 64];
+      if (PACK && 4 * kg >= M) continue;
+      auto quarters = [&](int at) __attribute__((always_inline)) {
+        float4v v = red[(rw * WR * MT + ij) * 64 + at];
 #pragma unroll
-      for (int q = 1; q < 4; ++q) v += red[((q * L::RW + rw) * WR * MT + ij) * 64];
+        for (int q = 1; q < 4; ++q) v += red[((q * L::RW + rw) * WR * MT + ij) * 64 + at];
+        return v;
+      };
+      float4v v;
+      if constexpr (!PACK) v = quarters(0);
+      else if constexpr (F32) v = quarters(32) + quarters(0);  // tile row m + 8 is 32 lanes on, m + 4 16
+      else v = quarters(32) + quarters(16) + quarters(0);
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int m = j * 16 + 4 * kg + r;
@@ -749,15 +771,15 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
   }
 }
 
-template <int QT, bool F32, int MT>
+template <int QT, bool F32, int MT, bool PACK = false>
 int launch_sk(const SkArgs& a, int cus, hipStream_t s, const char* who) {
-  using L = SkLayout<QT, F32, MT>;
+  using L = SkLayout<QT, F32, MT, PACK>;
   if constexpr (L::FITS) {
     static std::atomic<uint64_t> attr{0};
-    int st = lds_attr_once(attr, (const void*)qgemm_skinny<QT, F32, MT>, L::LDS, who);
+    int st = lds_attr_once(attr, (const void*)qgemm_skinny<QT, F32, MT, PACK>, L::LDS, who);
     if (st) return st;
     const int grid = std::min(a.tile0[a.ngroups] * a.KS, cus * (4 / L::RW));
-    qgemm_skinny<QT, F32, MT><<<(unsigned)grid, 64 * L::WV, L::LDS, s>>>(a);
+    qgemm_skinny<QT, F32, MT, PACK><<<(unsigned)grid, 64 * L::WV, L::LDS, s>>>(a);
     TM_LAUNCH_CHECK(who);
     return TIERMM_OK;
   }
@@ -766,6 +788,7 @@ int launch_sk(const SkArgs& a, int cus, hipStream_t s, const char* who) {
 template <int QT, bool F32>
 int launch_sk_mt(int mt, const SkArgs& a, int cus, hipStream_t s, const char* who) {
   switch (mt) {
+    case 0: return launch_sk<QT, F32, 1, true>(a, cus, s, who);
     case 1: return launch_sk<QT, F32, 1>(a, cus, s, who);
     case 2: return launch_sk<QT, F32, 2>(a, cus, s, who);
     default: return launch_sk<QT, F32, 3>(a, cus, s, who);
@@ -864,13 +887,20 @@ int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows,
                  const uint16_t* xparts, size_t pstride, size_t kt, float* Y, int ldy, int N, int K, float beta,
                  bool f32, void* ws, int cus, hipStream_t s, const char* who) {
   const int ks = n == 1 ? sk_splits((rows[0] + 15) / 16, N, K, cus) : 1;
-  // launches of up to SK_G groups with the same number of row tiles
-  for (int mt = 1, g0 = 0; mt <= SK_MT; g0 < n ? mt : (g0 = 0, ++mt)) {
+  // Parts are packed where that takes no further launch: where it leaves some groups of up to 16 rows
+  // for a launch of their own, that costs more (64 experts, hidden 2048, ffn 1408, us: 16 tokens
+  // 149 -> 157, 32 tokens 166 -> 176) than the packed ones gain.
+  bool packed = true;
+  for (int g = 0; g < n; ++g) packed = packed && (rows[g] <= sk_pack(f32) || rows[g] > 16);
+  // launches of up to SK_G groups with the same number of row tiles (0: one of packed parts)
+  for (int kind = 0, g0 = 0; kind <= SK_MT; g0 < n ? kind : (g0 = 0, ++kind)) {
+    const bool pack = kind == 0;
+    const int mt = std::max(kind, 1);
     SkArgs a{};
     a.Y = Y; a.rb = rb; a.ldy = ldy; a.N = N; a.K = K; a.KS = ks; a.beta = beta;
     int total = 0, last = 0;
     for (; g0 < n && a.ngroups < SK_G; ++g0) {
-      if ((rows[g0] + 15) / 16 != mt) continue;
+      if ((packed && rows[g0] <= 16 ? 0 : (rows[g0] + 15) / 16) != kind) continue;
       const int j = a.ngroups++;
       a.row0[j] = row0[g0];
       a.rows[j] = rows[g0];
@@ -889,11 +919,11 @@ int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows,
     uint16_t* sums = f32 && sk_mins(qt) ? (uint16_t*)(b + w.s) : nullptr;
     int32_t* xe = (int32_t*)(b + w.e);
     a.X = x; a.S = sums; a.xexp = xe; a.P = (float*)(b + w.p); a.ps = (size_t)rows[0] * N;
-    if (xparts) sk_relayout3<<<total, 256, 0, s>>>(xparts, pstride, kt, a, x);
-    else if (f32) sk_split2<<<total, 256, 0, s>>>(X, a, x, sums, xe);
-    else sk_split3<<<total, 256, 0, s>>>(X, a, x);
+    if (xparts) (pack ? sk_relayout3<true> : sk_relayout3<false>)<<<total, 256, 0, s>>>(xparts, pstride, kt, a, x);
+    else if (f32) (pack ? sk_split2<true> : sk_split2<false>)<<<total, 256, 0, s>>>(X, a, x, sums, xe);
+    else (pack ? sk_split3<true> : sk_split3<false>)<<<total, 256, 0, s>>>(X, a, x);
     TM_LAUNCH_CHECK(who);
-    int st = f32 ? launch_sk_qt<true>(qt, mt, a, cus, s, who) : launch_sk_qt<false>(qt, mt, a, cus, s, who);
+    int st = f32 ? launch_sk_qt<true>(qt, kind, a, cus, s, who) : launch_sk_qt<false>(qt, kind, a, cus, s, who);
     if (st) return st;
     if (ks > 1) {
       st = qgemm_splitk_sum(a.P, a.ps, ks, Y + (size_t)row0[0] * ldy, ldy, rows[0], N, beta, s, who);
