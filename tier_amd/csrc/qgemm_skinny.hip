@@ -108,7 +108,8 @@ __device__ __forceinline__ int group_of(const int* start, int n, int i) {
 }
 // Row, tile and row in the tile of the i-th row of the groups
 __device__ __forceinline__ int row_place(const SkArgs& p, int i, size_t& tile, int& m) {
-  const int g = __builtin_amdgcn_readfirstlane(group_of(p.first, p.ngroups, i)), q = i - p.first[g];
+  const int g = p.ngroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(group_of(p.first, p.ngroups, i));
+  const int q = i - p.first[g];
   tile = p.mt0[g] + (q >> 4);
   m = q & 15;
   return p.row0[g] + q;
@@ -117,7 +118,7 @@ __device__ __forceinline__ int row_place(const SkArgs& p, int i, size_t& tile, i
 // x-ref: the three fp16 parts (split3_fp_k, tier.cpp:869-870); one row per block.  K past the
 // row is zero up to a whole unit.
 template <bool PACK>
-__global__ __launch_bounds__(256) void sk_split3(const float* __restrict__ x, const SkArgs p,
+__global__ __launch_bounds__(1024) void sk_split3(const float* __restrict__ x, const SkArgs p,
                                                  uint16_t* __restrict__ X) {
   const int K = p.K, kp = (K + SK_UNIT - 1) / SK_UNIT * SK_UNIT;
   size_t tile;
@@ -125,7 +126,7 @@ __global__ __launch_bounds__(256) void sk_split3(const float* __restrict__ x, co
   const int row = row_place(p, (int)blockIdx.x, tile, m);
   const float* xr = x + (size_t)row * K;
   const bool al = ((uintptr_t)xr & 15) == 0;
-  for (int k = 8 * threadIdx.x; k < kp; k += 2048) {
+  for (int k = 8 * threadIdx.x; k < kp; k += 8 * blockDim.x) {
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (k < K) load8(xr + k, al, v);
     uint16_t h[3][8];
@@ -142,13 +143,13 @@ __global__ __launch_bounds__(256) void sk_split3(const float* __restrict__ x, co
 // The same fragments from parts that are split already (planes part_stride apart; kt > 0:
 // K-tiled over kt rows).
 template <bool PACK>
-__global__ __launch_bounds__(256) void sk_relayout3(const uint16_t* __restrict__ parts, size_t stride, size_t kt,
+__global__ __launch_bounds__(1024) void sk_relayout3(const uint16_t* __restrict__ parts, size_t stride, size_t kt,
                                                     const SkArgs p, uint16_t* __restrict__ X) {
   const int K = p.K, kp = (K + SK_UNIT - 1) / SK_UNIT * SK_UNIT;
   size_t tile;
   int m;
   const int row = row_place(p, (int)blockIdx.x, tile, m);
-  for (int k = 8 * threadIdx.x; k < kp; k += 2048) {
+  for (int k = 8 * threadIdx.x; k < kp; k += 8 * blockDim.x) {
     uint16_t h[3][8];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -166,9 +167,9 @@ __global__ __launch_bounds__(256) void sk_relayout3(const uint16_t* __restrict__
 // fp16 parts: lane (m, kg) of the unit's sum fragment holds the hi parts of sub-blocks
 // 4 kg .. 4 kg + 3, then their lo parts, for kg < 2, and zeros beyond.
 template <bool PACK>
-__global__ __launch_bounds__(256) void sk_split2(const float* __restrict__ x, const SkArgs p, uint16_t* __restrict__ X,
+__global__ __launch_bounds__(1024) void sk_split2(const float* __restrict__ x, const SkArgs p, uint16_t* __restrict__ X,
                                                  uint16_t* __restrict__ S, int32_t* __restrict__ xexp) {
-  __shared__ float red[4];
+  __shared__ float red[16];
   const int K = p.K, kp = (K + SK_UNIT - 1) / SK_UNIT * SK_UNIT;
   size_t tile;
   int m;
@@ -176,17 +177,21 @@ __global__ __launch_bounds__(256) void sk_split2(const float* __restrict__ x, co
   const float* xr = x + (size_t)row * K;
   const bool al = ((uintptr_t)xr & 15) == 0;
   float amax = 0.f;
-  for (int k = 8 * threadIdx.x; k < K; k += 2048) {
+  for (int k = 8 * threadIdx.x; k < K; k += 8 * blockDim.x) {
     float v[8];
     load8(xr + k, al, v);
 #pragma unroll
     for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[e]));
   }
-  amax = block_max_256(amax, red);
+#pragma unroll
+  for (int d = 32; d; d >>= 1) amax = fmaxf(amax, __shfl_xor(amax, d, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = amax;
+  __syncthreads();
+  for (unsigned i = 0; i < blockDim.x >> 6; ++i) amax = fmaxf(amax, red[i]);
   const int ex = x3s_exp(amax);
   const float sc = ldexpf(1.f, ex);
   if (threadIdx.x == 0) xexp[row] = ex;
-  for (int k = 8 * threadIdx.x; k < kp; k += 2048) {
+  for (int k = 8 * threadIdx.x; k < kp; k += 8 * blockDim.x) {
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (k < K) load8(xr + k, al, v);
     uint16_t h[2][8];
@@ -535,7 +540,7 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
     int grp, n0, kz, u0, u1;
   };
   auto item = [&](int i) __attribute__((always_inline)) {
-    const int b = i % nt_all, kz = i / nt_all, g = __builtin_amdgcn_readfirstlane(group_of(p.tile0, p.ngroups, b));
+    const int b = i % nt_all, kz = i / nt_all, g = p.ngroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(group_of(p.tile0, p.ngroups, b));
     return Item{g, (b - p.tile0[g]) * L::BN, kz, nu * kz / p.KS, nu * (kz + 1) / p.KS};
   };
   const int rbytes = (int)((long)p.K * D::UB / SK_UNIT);  // of a row
@@ -919,9 +924,14 @@ int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows,
     uint16_t* sums = f32 && sk_mins(qt) ? (uint16_t*)(b + w.s) : nullptr;
     int32_t* xe = (int32_t*)(b + w.e);
     a.X = x; a.S = sums; a.xexp = xe; a.P = (float*)(b + w.p); a.ps = (size_t)rows[0] * N;
-    if (xparts) (pack ? sk_relayout3<true> : sk_relayout3<false>)<<<total, 256, 0, s>>>(xparts, pstride, kt, a, x);
-    else if (f32) (pack ? sk_split2<true> : sk_split2<false>)<<<total, 256, 0, s>>>(X, a, x, sums, xe);
-    else (pack ? sk_split3<true> : sk_split3<false>)<<<total, 256, 0, s>>>(X, a, x);
+    // a whole row at once, 8 elements a thread: its time is the latency of its loads (with the group
+    // search skipped for one group, 256 threads -> this, a call in us: F32 q4_K 1024x4096 M = 2
+    // 16.0 -> 14.0, M = 37 21.7 -> 19.8; 14336x5120 M = 2 25.7 -> 24.5, M = 37 40.4 -> 39.5)
+    const int nu = (K + SK_UNIT - 1) / SK_UNIT;
+    const unsigned thr = (unsigned)std::min(1024, (nu * SK_UNIT + 511) / 512 * 64);
+    if (xparts) (pack ? sk_relayout3<true> : sk_relayout3<false>)<<<total, thr, 0, s>>>(xparts, pstride, kt, a, x);
+    else if (f32) (pack ? sk_split2<true> : sk_split2<false>)<<<total, thr, 0, s>>>(X, a, x, sums, xe);
+    else (pack ? sk_split3<true> : sk_split3<false>)<<<total, thr, 0, s>>>(X, a, x);
     TM_LAUNCH_CHECK(who);
     int st = f32 ? launch_sk_qt<true>(qt, kind, a, cus, s, who) : launch_sk_qt<false>(qt, kind, a, cus, s, who);
     if (st) return st;
