@@ -16,13 +16,13 @@
 //     the scales; the minima are one product with the sub-block sums of x);
 //   - x is split and laid out as operand fragments once, by a launch before.
 // Measured, all launches of a call, in us (fused kernel -> this one):
-//   F32, N = 14336, K = 5120:  q4_K M = 2  59.7 -> 27.7, M = 37  62.7 -> 40.6;
-//     q6_K M = 2  61.0 -> 33.9, M = 37  65.1 -> 49.6;  q8_0 M = 2  69.1 -> 35.3
-//   F32, N = 1024, K = 4096:  q4_K M = 2  22.9 -> 15.0, M = 48  24.5 -> 21.0
-//   x-ref, N = 14336, K = 5120:  q4_K M = 2  44.9 -> 27.7, M = 32  43.0 -> 32.5;
+//   F32, N = 14336, K = 5120:  q4_K M = 2  59.7 -> 24.5, M = 37  62.7 -> 39.5;
+//     q6_K M = 2  61.0 -> 32.5, M = 37  65.1 -> 46.0;  q8_0 M = 2  69.1 -> 31.4
+//   F32, N = 1024, K = 4096:  q4_K M = 2  22.9 -> 14.0
+//   x-ref, N = 14336, K = 5120 (before the parts were packed):  q4_K M = 2  44.9 -> 27.7, M = 32  43.0 -> 32.5;
 //     q6_K M = 16  54.1 -> 34.6;  q8_0 M = 16  62.6 -> 41.5
 // with errors against fp64 no larger (F32 q4_K 5.6e-7 -> 4.6e-7, q6_K 5.6e-7 -> 1.2e-7).  What
-// is left over the weights' read (7 us at q4_K) is the split and reduce launches (10 us), the
+// is left over the weights' read (8 us at q4_K) is the split and reduce launches (9 us), the
 // first unit's latency and, per unit, decode, MFMAs and LDS reads that overlap in part.
 #include <algorithm>
 
@@ -540,7 +540,8 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
     int grp, n0, kz, u0, u1;
   };
   auto item = [&](int i) __attribute__((always_inline)) {
-    const int b = i % nt_all, kz = i / nt_all, g = p.ngroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(group_of(p.tile0, p.ngroups, b));
+    const int b = i % nt_all, kz = i / nt_all;
+    const int g = p.ngroups == 1 ? 0 : __builtin_amdgcn_readfirstlane(group_of(p.tile0, p.ngroups, b));
     return Item{g, (b - p.tile0[g]) * L::BN, kz, nu * kz / p.KS, nu * (kz + 1) / p.KS};
   };
   const int rbytes = (int)((long)p.K * D::UB / SK_UNIT);  // of a row
