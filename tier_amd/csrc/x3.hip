@@ -1080,6 +1080,20 @@ int big_group_chunk(const int* offs, int n_experts, int N, int K) {
 
 }  // namespace
 
+// Products below the big-tile kernel: 128 x 128 tiles where they come near filling the 256 CUs, else
+// 64 x 64 ones, four times as many (each output is summed in the same order: the same bits).  With
+// two workgroups or more on a CU the loads of one cover the other's products, which one 128-tile
+// workgroup on some of the CUs cannot.  Whole calls on f16 rows, 128 -> 64 tiles, us: 5120x4096
+// M = 2 110 -> 59, M = 203 (80 tiles) 114 -> 73, M = 512 (160 tiles) 118 -> 109; 5120x14336 M = 512
+// 558 -> 437; 1024x5120 M = 512 149 -> 88.  At 224 tiles the 128-wide ones win: 14336x5120 M = 203
+// 166, 64-wide 202.
+template <int MODE>
+int launch_x3_small(const X3Args& a, hipStream_t s, const char* who) {
+  const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
+  if (tiles <= 160) return launch_x3<64, 64, MODE>(a, s, who);
+  return launch_x3<128, 128, MODE>(a, s, who);
+}
+
 // x3-ref product on pre-split activations: C[M][ldc] (beta)= sum_parts Xpart[M][K] * W[N][K]^T,
 // parts at xparts + {0, stride, 2*stride} in HML order, W fp16 with row stride ldw.
 int x3ref_nt(const uint16_t* xparts, size_t stride, const uint16_t* W, int ldw, float* C, int ldc, int M, int N,
@@ -1101,10 +1115,10 @@ int x3ref_nt(const uint16_t* xparts, size_t stride, const uint16_t* W, int ldw, 
   a.beta = beta;
   if (bf16) {
     if (big_tiles(M, N) >= 192) return launch_x3_big<X3_REF_BF16>(a, s, who);
-    return launch_x3<128, 128, X3_REF_BF16>(a, s, who);
+    return launch_x3_small<X3_REF_BF16>(a, s, who);
   }
   if (big_tiles(M, N) >= 192) return launch_x3_big<X3_REF>(a, s, who);
-  return launch_x3<128, 128, X3_REF>(a, s, who);
+  return launch_x3_small<X3_REF>(a, s, who);
 }
 
 // Rows held in registers where they fit (one read of the source), else two passes.
