@@ -127,3 +127,38 @@ def test_few_rows_in_a_workspace_of_the_general_path(gpu, t, M, N, K, mode):
         T.qgemm(W.ptr, t, T.q_row_bytes(t, K), X.ptr, Y.ptr, M, N, K, mode=mode, ws=ws.ptr, ws_bytes=size)
         hip.synchronize()
         assert _err(Y.download(np.float32, M * N).reshape(M, N), x.astype(np.float64) @ w.T, x, w) <= BAR
+
+
+@pytest.mark.parametrize("types,sizes,N,K", [
+    ([T.Q4_K], [16], 2816, 2048), ([T.Q4_K] * 64, [0] * 37 + [1] + [0] * 26, 2816, 2048),
+    ([T.Q5_0] * 3, [0, 5, 0], 600, 1408), ([T.Q4_K, T.Q6_K, T.Q4_K], [3, 20, 0], 1024, 4096)],
+    ids=["one", "one_of_64", "one_short_k", "one_of_each_type"])
+def test_few_rows_one_routed_expert(gpu, types, sizes, N, K):
+    """One expert of a type has rows: its product stays inside a workspace of exactly the queried size
+    (it may not split K, whose partial sums that size does not hold), and its bits are those that it
+    has beside a second expert of its type."""
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    P = int(offs[-1])
+    x = activations(P, K, seed=N)
+    made = {t: _weight(t, N, K, 11 + t, oracle.OUT_F16) for t in set(types)}
+    bufs = {t: hip.to_device(made[t][0]) for t in made}
+
+    def run(types, offs, x):
+        need, guard = T.qgemm_grouped_ws_bytes(types, offs.tolist(), N, K), 8 << 20
+        X, Y, ws = hip.to_device(x), hip.DeviceBuffer(x.shape[0] * N * 4), hip.DeviceBuffer(need + guard)
+        ws.fill_bytes(0x5a)
+        T.qgemm_grouped([bufs[t].ptr for t in types], types, [T.q_row_bytes(t, K) for t in types], X.ptr, offs, Y.ptr,
+                        N, K, ws=ws.ptr, ws_bytes=need)
+        hip.synchronize()
+        assert np.all(ws.download(np.uint8, guard, need) == 0x5a)
+        return Y.download(np.float32, x.shape[0] * N).reshape(-1, N)
+
+    got = run(types, offs, x)
+    for e, t in enumerate(types):
+        r = slice(offs[e], offs[e + 1])
+        if sizes[e]:
+            w = made[t][1]
+            assert _err(got[r], x[r].astype(np.float64) @ w.T, x[r], w) <= BAR, e
+    beside = run(types + types, np.concatenate([offs, offs[1:] + P]).astype(np.int32), np.concatenate([x, x]))
+    assert np.array_equal(beside[:P].view(np.uint32), got.view(np.uint32))
+    assert np.array_equal(beside[P:].view(np.uint32), got.view(np.uint32))

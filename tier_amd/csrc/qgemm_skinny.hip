@@ -888,11 +888,14 @@ int qgemm_splitk_sum(const float* P, size_t ps, int ks, float* Y, int ldy, int r
 
 // n groups (rows[g] > 0 rows of x and Y from row0[g], weight W[g] of type qt).  xparts given:
 // x comes split in three parts (x3-ref, one group), parts pstride apart, K-tiled over kt
-// rows when kt > 0; otherwise X is split here.
+// rows when kt > 0; otherwise X is split here.  split (one group): K may be split, and ws holds
+// qgemm_skinny_ws_bytes; else qgemm_skinny_group_ws_bytes, which has no room for partial sums -- a
+// routed batch in which one expert of a type has rows is a group of one, and must not split either
+// (its rows would be summed in another order than beside other experts, too).
 int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows, int n, size_t rb, const float* X,
                  const uint16_t* xparts, size_t pstride, size_t kt, float* Y, int ldy, int N, int K, float beta,
-                 bool f32, void* ws, int cus, hipStream_t s, const char* who) {
-  const int ks = n == 1 ? sk_splits((rows[0] + 15) / 16, N, K, cus) : 1;
+                 bool f32, bool split, void* ws, size_t ws_bytes, int cus, hipStream_t s, const char* who) {
+  const int ks = split && n == 1 ? sk_splits((rows[0] + 15) / 16, N, K, cus) : 1;
   // Parts are packed where that takes no further launch: where it leaves some groups of up to 16 rows
   // for a launch of their own, that costs more (64 experts, hidden 2048, ffn 1408, us: 16 tokens
   // 149 -> 157, 32 tokens 166 -> 176) than the packed ones gain.
@@ -920,6 +923,8 @@ int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows,
     }
     if (!a.ngroups) continue;
     const SkWs w = sk_ws(qt, (size_t)a.mtot, (size_t)last, N, K, f32, ks);
+    if (w.total > ws_bytes)
+      return set_error(TIERMM_EINVAL, "%s: few-row workspace of %zu bytes, %zu needed", who, ws_bytes, w.total);
     uint8_t* b = (uint8_t*)ws;
     uint16_t* x = (uint16_t*)(b + w.x);
     uint16_t* sums = f32 && sk_mins(qt) ? (uint16_t*)(b + w.s) : nullptr;

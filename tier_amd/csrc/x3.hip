@@ -56,7 +56,7 @@ size_t qgemm_skinny_group_ws_bytes(int qt, const int* rows, int n, int N, int K)
 size_t qgemm_skinny_routed_ws_bytes(size_t P, int n, int K);
 int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows, int n, size_t rb, const float* X,
                  const uint16_t* xparts, size_t pstride, size_t kt, float* Y, int ldy, int N, int K, float beta, bool f32,
-                 void* ws, int cus, hipStream_t s, const char* who);
+                 bool split, void* ws, size_t ws_bytes, int cus, hipStream_t s, const char* who);
 int cus_or_default();
 
 namespace {
@@ -1559,8 +1559,8 @@ int tiermm_qgemm(const void* W, int qtype, size_t rb, const float* X, float* Y, 
     st = device_cus(&cus);
     if (st) return st;
     const int row0 = 0;
-    return qgemm_skinny(&W, qtype, &row0, &M, 1, rb, X, nullptr, 0, 0, Y, ldy, N, K, beta, mode == TIERMM_MODE_F32, w, cus,
-                        s, who);
+    return qgemm_skinny(&W, qtype, &row0, &M, 1, rb, X, nullptr, 0, 0, Y, ldy, N, K, beta, mode == TIERMM_MODE_F32, true,
+                        w, few, cus, s, who);
   }
   if (mode == TIERMM_MODE_F32 && qgemm_fusable(qtype, &M, 1, N, K, true, true)) {
     // the same semantics with W decoded inside the GEMM: no fp32 or fp16 copy of W
@@ -1684,7 +1684,7 @@ int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xp
     if (st) return st;
     const int row0 = 0;
     return qgemm_skinny(&W, qtype, &row0, &M, 1, rb, nullptr, xparts, part_stride, tiled ? (size_t)M : 0, Y, ldy, N, K, beta,
-                        false, w, cus, s, who);
+                        false, true, w, few, cus, s, who);
   }
   if (qgemm_fusable(qtype, &M, 1, N, K, true)) {
     int cus = 0;
@@ -1811,7 +1811,7 @@ int tiermm_qgemm_grouped(const void* const* W_e, const int* qtype_e, const size_
       const auto& g = gs[i];
       if (!g.same_rb) return set_error(TIERMM_EINVAL, "%s: experts of one type with different row bytes", who);
       st = qgemm_skinny(g.W.data(), types[i].first, g.row0.data(), g.rows.data(), (int)g.rows.size(), g.rb, X_sorted,
-                        nullptr, 0, 0, Y_sorted, N, N, K, 0.f, false, w, cus, s, who);
+                        nullptr, 0, 0, Y_sorted, N, N, K, 0.f, false, false, w, few, cus, s, who);
       if (st) return st;
     }
     return TIERMM_OK;
