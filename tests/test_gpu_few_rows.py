@@ -162,3 +162,47 @@ def test_few_rows_one_routed_expert(gpu, types, sizes, N, K):
     beside = run(types + types, np.concatenate([offs, offs[1:] + P]).astype(np.int32), np.concatenate([x, x]))
     assert np.array_equal(beside[:P].view(np.uint32), got.view(np.uint32))
     assert np.array_equal(beside[P:].view(np.uint32), got.view(np.uint32))
+
+
+def _shifted(kind, M, K, seed):
+    """Rows of x whose mean outweighs their spread, and rows of few distinct values."""
+    n = activations(M, K, seed)
+    c = np.exp(activations(M, 1, seed + 1))
+    x = {"constant": np.broadcast_to(np.linspace(0.1, 3.0, M)[:, None], (M, K)), "two": np.where(n > 0, 0.1, 0.3),
+         "near_one": 1 + 0.01 * n, "scaled": c * (1 + 0.3 * n), "three": 3 + n, "abs": np.abs(n)}[kind]
+    return np.ascontiguousarray(x, np.float32)
+
+
+@pytest.mark.parametrize("kind", ["constant", "two", "near_one", "scaled", "three", "abs"])
+@pytest.mark.parametrize("M", [1, 8, 9, 37, 48])
+@pytest.mark.parametrize("t", [T.Q4_K, T.Q5_K])
+def test_few_rows_f32_shifted_x(gpu, monkeypatch, t, M, kind):
+    """F32 where x does not average out: codes and minima of q4_K / q5_K are each several times the
+    weight, so their products with x may not be rounded apart.  Every row within 2^-20, and no further
+    off than the tiled kernel, which multiplies the weights themselves (TIERMM_QGEMM_TILE asks for it)."""
+    N, K = 300, 5120
+    blocks, w = _weight(t, N, K, 21 + t, oracle.OUT_F32)
+    x = _shifted(kind, M, K, M + t)
+    want = x.astype(np.float64) @ w.T
+    rows = lambda y: np.linalg.norm(y - want, axis=1) / np.linalg.norm(want, axis=1)  # noqa: E731
+    got = _run(blocks, t, x, N, K, T.MODE_F32)
+    monkeypatch.setenv("TIERMM_QGEMM_TILE", "-")
+    tiled = _run(blocks, t, x, N, K, T.MODE_F32)
+    assert rows(got).max() <= BAR
+    assert oracle.rel_fro(got, want) <= oracle.rel_fro(tiled, want)
+
+
+@pytest.mark.parametrize("t", [T.Q4_K, T.Q5_K])
+def test_few_rows_nonfinite_kq_scales(gpu, t):
+    """q4_K / q5_K, d or dmin infinite or NaN: that weight row's outputs are NaN, the others finite."""
+    M, N, K = 20, 40, 512
+    blocks, w = _weight(t, N, K, 29 + t, oracle.OUT_F32)
+    b = blocks.reshape(N, -1, oracle.block(t)[1]).copy()
+    rows = (3, 8, 11, 17, 30, 39)
+    for i, row in enumerate(rows):  # d (bytes 0, 1) and dmin (2, 3) of either super-block
+        b[row, i // 3, 2 * (i % 2):2 * (i % 2) + 2] = np.array([(0x7c00, 0xfc00, 0x7e00)[i % 3]], np.uint16).view(np.uint8)
+    x = activations(M, K, seed=t)
+    y = _run(b.reshape(N, -1), t, x, N, K, T.MODE_F32)
+    bad = np.isin(np.arange(N), rows)
+    assert np.all(np.isnan(y[:, bad]))
+    assert oracle.rel_fro(y[:, ~bad], (x.astype(np.float64) @ w.T)[:, ~bad]) <= BAR

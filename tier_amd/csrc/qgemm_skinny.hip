@@ -13,7 +13,11 @@
 //   - codes are read as fp16 subnormals (no conversions), and for F32 the block scale is applied
 //     to the sums where the code times its sub-block scale is a whole number that fp16 holds
 //     (q4_K, q5_K: two products, x hi and lo, where the fused kernel has three, and no pass over
-//     the scales; the minima are one product with the sub-block sums of x);
+//     the scales).  The codes are centred, d sc q - dmin m = d sc (q - c) + (c d sc - dmin m), c = 8
+//     or 16, and the second term, one fp32 factor a sub-block, is one product with the sub-block
+//     sums of the split x.  With the codes as they are the two terms are each several times their
+//     difference, and what rounds in either stays: q4_K 300x5120, M = 37, rows of x that are
+//     constant 1.1e-5 off 64 bits -> 2.8e-7, 3 + n 1.2e-6 -> 2.1e-7 (fused kernel 4.0e-7);
 //   - x is split and laid out as operand fragments once, by a launch before.
 // Measured, all launches of a call, in us (fused kernel -> this one):
 //   F32, N = 14336, K = 5120:  q4_K M = 2  59.7 -> 24.5, M = 37  62.7 -> 39.5;
@@ -21,7 +25,7 @@
 //   F32, N = 1024, K = 4096:  q4_K M = 2  22.9 -> 14.0
 //   x-ref, N = 14336, K = 5120 (before the parts were packed):  q4_K M = 2  44.9 -> 27.7, M = 32  43.0 -> 32.5;
 //     q6_K M = 16  54.1 -> 34.6;  q8_0 M = 16  62.6 -> 41.5
-// with errors against fp64 no larger (F32 q4_K 5.6e-7 -> 4.6e-7, q6_K 5.6e-7 -> 1.2e-7).  What
+// with errors against fp64 no larger (F32 q4_K, N(0, 1): 4.0e-7 -> 1.4e-7).  What
 // is left over the weights' read (8 us at q4_K) is the split and reduce launches (9 us), the
 // first unit's latency and, per unit, decode, MFMAs and LDS reads that overlap in part.
 #include <algorithm>
@@ -35,6 +39,7 @@ int device_cus(int* cus);
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 h2v __attribute__((ext_vector_type(2)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
@@ -55,7 +60,7 @@ constexpr int SK_UNIT = 256;      // K per step of the K loop (8 MFMA steps of 3
 
 struct SkArgs {
   const uint16_t* X;  // fragments [unit][step 8][part][tile][64 lanes][8 halfs]
-  const uint16_t* S;  // F32, formats with minima: sub-block sums [unit][tile][64][8]
+  const uint16_t* S;  // F32, formats with minima: sub-block sums [unit][tile][t 2][64 lanes][4 halfs]
   float* Y;
   float* P;           // KS > 1: partial sums of split z at P + z * ps, rows of N floats
   const int32_t* xexp;
@@ -163,9 +168,9 @@ __global__ __launch_bounds__(1024) void sk_relayout3(const uint16_t* __restrict_
 }
 
 // F32: the two-part split with a power of two per row (x3s_split's), and with S the
-// sub-block sums S_b = sum of x * 2^e over the 32 elements of sub-block b, over 32, in two
-// fp16 parts: lane (m, kg) of the unit's sum fragment holds the hi parts of sub-blocks
-// 4 kg .. 4 kg + 3, then their lo parts, for kg < 2, and zeros beyond.
+// sub-block sums S_b = sum of hi + lo (what the products see of x) over the 32 elements of
+// sub-block b, over 32, in two fp16 parts: lane (m, kg) of the unit's sum fragment t holds
+// hi, hi, lo, lo of sub-block b = 4 (kg % 2) + 2 (kg / 2) + t.
 template <bool PACK>
 __global__ __launch_bounds__(1024) void sk_split2(const float* __restrict__ x, const SkArgs p, uint16_t* __restrict__ X,
                                                  uint16_t* __restrict__ S, int32_t* __restrict__ xexp) {
@@ -195,30 +200,27 @@ __global__ __launch_bounds__(1024) void sk_split2(const float* __restrict__ x, c
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (k < K) load8(xr + k, al, v);
     uint16_t h[2][8];
-    float sum = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
       const float f = v[e] * sc;
       h[0][e] = f2h(f);
       h[1][e] = f2h(f - h2f(h[0][e]));
-      sum += f;
+      v[e] = h2f(h[0][e]) + h2f(h[1][e]);  // exact
     }
     put_frag<2, true, PACK>(X, p.mtot, tile, m, k, h);
-    if (S) {  // four neighbouring lanes hold a sub-block
+    if (S) {  // four neighbouring lanes hold a sub-block; in pairs, so that equal values add without rounding
+      float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
       sum += __shfl_xor(sum, 1, 64);
       sum += __shfl_xor(sum, 2, 64);
       sum *= 0.03125f;
-      const uint16_t s0 = f2h(sum), s1 = f2h(sum - h2f(s0));
-      const int b = (k >> 5) & 7;
+      const uint32_t s0 = f2h(sum), s1 = f2h(sum - h2f((uint16_t)s0));
+      const int b = (k >> 5) & 7, kg = 2 * ((b >> 1) & 1) + (b >> 2);
       uint16_t* f = S + ((size_t)(k >> 8) * p.mtot + tile) * 512;
       if ((k & 31) == 0) {
-        f[(16 * (b >> 2) + m) * 8 + (b & 3)] = s0;
-        f[(16 * (b >> 2) + m) * 8 + 4 + (b & 3)] = s1;
+        u32x2* o = (u32x2*)(f + 256 * (b & 1) + (16 * kg + m) * 4);
+        *o = u32x2{s0 * 0x10001u, s1 * 0x10001u};
+        if (PACK) o[sk_pack(true)] = u32x2{0, 0};  // the sums count once, with the hi parts
       }
-      if ((k & 255) == 16 || (k & 255) == 24) *(u32x4*)(f + (16 * ((k & 255) >> 3) + m) * 8) = u32x4{0, 0, 0, 0};
-      // the sums count once, with the hi parts
-      if (PACK && (k & 255) >= 32 && (k & 255) < 64)
-        *(u32x4*)(f + (16 * (((k & 255) - 32) >> 3) + m + sk_pack(true)) * 8) = u32x4{0, 0, 0, 0};
     }
   }
 }
@@ -295,15 +297,23 @@ __device__ __forceinline__ uint32_t kq_bytes(u32x4 h, int kh) {
   const uint32_t lo = MIN ? h[2] : h[1];
   return kh ? ((h[3] >> (MIN ? 4 : 0)) & 0x0f0f0f0fu) | ((lo >> 2) & 0x30303030u) : lo & 0x3f3f3f3fu;
 }
-// q4_K / q5_K: 32 times the minima of the quarter's two sub-blocks, against the sums' hi and lo
-// parts, in the lanes kg == kh (zero in the other places)
-__device__ __forceinline__ u32x4 kq_mins(u32x4 h, int kh, int t, int kg) {
-  const uint32_t b = kg == kh ? kq_bytes<true>(h, kh) & (0x00ff00ffu << (8 * t)) : 0u;
-  // 1024 + m in fp16, times 32, less 32768
-  const h2v k = dup(32.f), c = dup(-32768.f);
-  const uint32_t m0 = as_u(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0x64646464u, b, 0x07010700u)), k, c));
-  const uint32_t m1 = as_u(__builtin_elementwise_fma(as_h2(__builtin_amdgcn_perm(0x64646464u, b, 0x07030702u)), k, c));
-  return u32x4{m0, m1, m0, m1};
+// q4_K / q5_K, codes centred by C: the factor C d sc - dmin m of this lane's sub-block in two fp16
+// parts, times a power of two that keeps it below 2^15 (126 max(C |d|, |dmin|) bounds it), against
+// the hi and lo sums, in the lanes kg % 2 == kh and zero in the others; inv = 32 over that power,
+// which takes the product to the factor's own scale
+template <int C>
+__device__ __forceinline__ u32x2 kq_offset(u32x4 h, int kh, int t, int kg, float& inv) {
+  const int sh = 16 * (kg >> 1) + 8 * t;
+  const float cd = (float)C * h2f(h[0] & 0xffffu), dm = h2f(h[0] >> 16);
+  const float m = dm * (float)((kq_bytes<true>(h, kh) >> sh) & 0xffu);  // exact
+  const float b = fmaf(cd, (float)((kq_bytes<false>(h, kh) >> sh) & 0xffu), -m);
+  // the exponent is 0 for 0, Inf and NaN; non-finite factors stay so
+  const int e = 8 - __builtin_amdgcn_frexp_expf(fmaxf(fabsf(cd), fabsf(dm)));
+  inv = ldexpf(32.f, -e);
+  const float v = ldexpf(b, e);
+  const uint32_t hi = f2h(v), lo = f2h(v - h2f((uint16_t)hi));
+  const uint32_t w = (kg & 1) == kh ? hi | lo << 16 : 0u;
+  return u32x2{w, w};
 }
 
 template <>
@@ -325,19 +335,21 @@ struct Sk<QT_Q4_K> {
 #pragma unroll
       for (int k = 0; k < 4; ++k) mix4((q[k] >> (4 * t)) & 0x0f0f0f0fu, dsc * 0x1p24f, -dm, o[2 * k], o[2 * k + 1]);
     } else {
-      // sc * q * 2^-14, sc * q at most 945: exact.  q as a subnormal times sc * 2^10
-      const h2v a = dup((float)(sc << 10));
+      // sc (q - 8) 2^-14, sc |q - 8| at most 504: exact.  q as a subnormal times sc 2^10, less 8 sc 2^-14
+      const h2v a = dup((float)(sc << 10)), z = dup((float)sc * -0x1p-11f);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        o[2 * k] = as_u(as_h2((q[k] >> (4 * t)) & 0x000f000fu) * a);
-        o[2 * k + 1] = as_u(as_h2((q[k] >> (8 + 4 * t)) & 0x000f000fu) * a);
+        o[2 * k] = as_u(__builtin_elementwise_fma(as_h2((q[k] >> (4 * t)) & 0x000f000fu), a, z));
+        o[2 * k + 1] = as_u(__builtin_elementwise_fma(as_h2((q[k] >> (8 + 4 * t)) & 0x000f000fu), a, z));
       }
     }
   }
   __device__ __forceinline__ float norm() const { return 1.f; }
-  __device__ __forceinline__ float post(float) const { return or_nan(h2f(h[0] & 0xffffu) * 0x1p14f); }
-  __device__ __forceinline__ u32x4 mins(int kh, int t, int kg) const { return kq_mins(h, kh, t, kg); }
-  __device__ __forceinline__ float dmin() const { return or_nan(h2f(h[0] >> 16)); }
+  // (a d that is not finite makes the offset's parts, and the row, NaN)
+  __device__ __forceinline__ float post(float) const { return h2f(h[0] & 0xffffu) * 0x1p14f; }
+  __device__ __forceinline__ u32x2 offset(int kh, int t, int kg, float& inv) const {
+    return kq_offset<8>(h, kh, t, kg, inv);
+  }
 };
 
 template <>
@@ -362,19 +374,21 @@ struct Sk<QT_Q5_K> {
       const float dsc = h2f(h[0] & 0xffffu) * (float)sc, dm = h2f(h[0] >> 16) * (float)mn;
 #pragma unroll
       for (int k = 0; k < 4; ++k) mix4(v[k], dsc * 0x1p24f, -dm, o[2 * k], o[2 * k + 1]);
-    } else {  // sc * q * 2^-14, sc * q at most 1953: exact
-      const h2v a = dup((float)(sc << 10));
+    } else {  // sc (q - 16) 2^-14, sc |q - 16| at most 1008: exact
+      const h2v a = dup((float)(sc << 10)), z = dup((float)sc * -0x1p-10f);
 #pragma unroll
       for (int k = 0; k < 4; ++k) {
-        o[2 * k] = as_u(as_h2(v[k] & 0x00ff00ffu) * a);
-        o[2 * k + 1] = as_u(as_h2((v[k] >> 8) & 0x00ff00ffu) * a);
+        o[2 * k] = as_u(__builtin_elementwise_fma(as_h2(v[k] & 0x00ff00ffu), a, z));
+        o[2 * k + 1] = as_u(__builtin_elementwise_fma(as_h2((v[k] >> 8) & 0x00ff00ffu), a, z));
       }
     }
   }
   __device__ __forceinline__ float norm() const { return 1.f; }
-  __device__ __forceinline__ float post(float) const { return or_nan(h2f(h[0] & 0xffffu) * 0x1p14f); }
-  __device__ __forceinline__ u32x4 mins(int kh, int t, int kg) const { return kq_mins(h, kh, t, kg); }
-  __device__ __forceinline__ float dmin() const { return or_nan(h2f(h[0] >> 16)); }
+  // (a d that is not finite makes the offset's parts, and the row, NaN)
+  __device__ __forceinline__ float post(float) const { return h2f(h[0] & 0xffffu) * 0x1p14f; }
+  __device__ __forceinline__ u32x2 offset(int kh, int t, int kg, float& inv) const {
+    return kq_offset<16>(h, kh, t, kg, inv);
+  }
 };
 
 template <>
@@ -713,18 +727,16 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
 #pragma unroll
         for (int i = 0; i < WR; ++i) {
           float s = cur[i].post(nm[i]);
-          asm volatile("" : "+v"(s));  // (else the NaN select moves behind each product)
+          if constexpr (!L::MINS) asm volatile("" : "+v"(s));  // (else the NaN select moves behind each product)
           if constexpr (L::MINS) {
-            // codes and minima of the same elements nearly cancel: with each other first, then into the sum
-            const half8 mn = __builtin_bit_cast(half8, cur[i].mins(kh, t, kg));
-            float dm = cur[i].dmin();
-            asm volatile("" : "+v"(dm));
+            float inv;
+            const half4 off = __builtin_bit_cast(half4, cur[i].offset(kh, t, kg, inv));
 #pragma unroll
             for (int j = 0; j < MT; ++j) {
-              const half8 a = *(const half8*)(xs + (8 * NP * MT + j) * 1024);
-              const float4v m = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, mn, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+              const half4 a = *(const half4*)(xs - lane * 8 + (8 * NP * MT + j) * 1024 + t * 512);
+              const float4v m = __builtin_amdgcn_mfma_f32_16x16x16f16(a, off, float4v{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
 #pragma unroll
-              for (int r = 0; r < 4; ++r) acc[i][j][r] += fmaf(c[i][j][r], s, -(m[r] * dm));
+              for (int r = 0; r < 4; ++r) acc[i][j][r] = fmaf(c[i][j][r], s, fmaf(m[r], inv, acc[i][j][r]));
             }
           } else {
 #pragma unroll
