@@ -69,3 +69,63 @@ def test_dot_gemv_nonfinite_scale(gpu, t):
     ok = np.isfinite(want)
     assert ok.sum() == N - 3
     assert oracle.rel_fro(y[ok], oracle.gemv_f64(blocks, t, x, N, K)[ok]) <= 2e-6
+
+
+def _zero_at(t, b, j):
+    """Element j < 16 of each 32-element block (of each 256-element one, for the K types) set to weight 0."""
+    b = b.copy()
+    if t == T.Q4_0:
+        b[..., 2 + j] = b[..., 2 + j] & 0xf0 | 8
+    elif t == T.Q4_1:  # m = -8 d
+        d = b[..., 0:2].copy().view(np.float16)
+        b[..., 2:4] = (d * np.float16(-8)).view(np.uint8)
+        b[..., 4 + j] = b[..., 4 + j] & 0xf0 | 8
+    elif t == T.Q5_0:
+        b[..., 2 + j // 8] |= 1 << (j % 8)
+        b[..., 6 + j] &= 0xf0
+    elif t == T.Q5_1:  # m = -16 d
+        d = b[..., 0:2].copy().view(np.float16)
+        b[..., 2:4] = (d * np.float16(-16)).view(np.uint8)
+        b[..., 4 + j // 8] |= 1 << (j % 8)
+        b[..., 8 + j] &= 0xf0
+    elif t == T.Q8_0:
+        b[..., 2 + j] = 0
+    elif t == T.Q2_K:  # d sc 1 - dmin m, with dmin = d and m = sc
+        b[..., :16] = (b[..., :16] & 15) * 17
+        b[..., 82:84] = b[..., 80:82]
+        b[..., 16 + j] = b[..., 16 + j] & 0xfc | 1
+    elif t == T.Q3_K:
+        b[..., j] |= 1
+        b[..., 32 + j] &= 0xfc
+    elif t == T.Q6_K:
+        b[..., j] &= 0xf0
+        b[..., 128 + j] = b[..., 128 + j] & 0xfc | 2
+    return b
+
+
+@pytest.mark.parametrize("mag", [64.0, 2.0 ** 40])
+@pytest.mark.parametrize("t", [T.Q4_0, T.Q4_1, T.Q5_0, T.Q5_1, T.Q8_0, T.Q2_K, T.Q3_K, T.Q6_K])
+def test_dot_gemv_outlier_in_x(gpu, t, mag):
+    """An outlier of x where every row's weight is zero, beside ordinary values: its block's other
+    elements keep the bits that fp32 sums would give them.  Outliers in every block and in every third."""
+    be, bb = oracle.block(t)
+    for N, K, step in ((40, 1280, 1), (257, 14336, 3), (1000, 2304, 1)):
+        blocks, x = _blocks(t, N, K, 5 * N + t)
+        b = _zero_at(t, blocks.reshape(N, -1, bb), 5).reshape(N, -1)
+        at = np.arange(5, K, be)[::step]
+        assert np.all(oracle.dequant(b, t, K, oracle.OUT_F32).reshape(N, K)[:, at] == 0)
+        x[at] = mag * np.where(np.arange(at.size) % 2, 1, -1)
+        rest = x.copy()
+        rest[at] = 0
+        y = _run(b, t, x, N, K)
+        assert oracle.rel_fro(y, oracle.gemv_f64(b, t, rest, N, K)) <= 2e-6, (N, K)
+
+
+@pytest.mark.parametrize("t", SMALL + SUPER)
+def test_dot_gemv_tiny_x(gpu, t):
+    """x of 2^-114: beyond the exponent that scales the digits to full width."""
+    N, K = 40, 5376
+    blocks, x = _blocks(t, N, K, 31 + t)
+    x *= np.float32(2.0 ** -114)
+    y = _run(blocks, t, x, N, K).astype(np.float64) * 2.0 ** 114
+    assert oracle.rel_fro(y, oracle.gemv_f64(blocks, t, x, N, K) * 2.0 ** 114) <= 2e-6
