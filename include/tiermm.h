@@ -259,8 +259,9 @@ size_t tiermm_sgemm_ws_bytes(int opA, int m, int n, int k);
  * tiermm_dequant.  The workspace (tiermm_qgemm_ws_bytes) holds the x parts and,
  * for q8_0 / q4_K / q5_K / q6_K / q5_0 (decoded inside the GEMM), the split-K partial
  * sums, or for the other types the fp16 weight; a call of few rows whose workspace
- * (sized for another M) has no room for the few-row kernel's sums takes the tiled
- * kernel.  The environment variable
+ * has no room for the few-row kernel's sums takes the tiled kernel (TIERMM_MODE_F32: so
+ * may one sized for more than 48 rows; an X3REF size holds the sums of any fewer rows).
+ * The environment variable
  * TIERMM_QGEMM_TILE="BN,KS[,KC]" overrides the fused kernel's tile width, split count
  * and accumulation chunks (read at each call, and by the size query; ignored when
  * invalid for the shape). */
@@ -285,7 +286,8 @@ int tiermm_qgemm_plan(int qtype, int M, int N, int K, int* bn, int* ks, int* kc)
  *                          is one contiguous kilobyte, the layout tiermm_qgemm uses
  *                          itself, and the faster one.
  * K a multiple of 32 (TIERMM_UNSUPPORTED otherwise).  Same result, bit for bit, as
- * tiermm_qgemm on the unsplit x.  Workspace (tiermm_qgemm_x3parts_ws_bytes): the fused
+ * tiermm_qgemm on the unsplit x, each in a workspace of at least its size query (or both
+ * in the pool).  Workspace (tiermm_qgemm_x3parts_ws_bytes): the fused
  * kernel's split-K partial sums, or the fp16 weight for the types it does not decode. */
 #define TIERMM_PARTS_ROWS 0
 #define TIERMM_PARTS_KTILED 1

@@ -1,7 +1,8 @@
 """Workspace sizes of products with few rows, on the host: a routed batch's size holds for every
 routing of as many rows to as many experts, and a small M's is no less than what the general path,
 to which the few-row kernel leaves a call that has no room for its own, needs (TIERMM_QGEMM_TILE
-asks for that path)."""
+asks for that path), and an x3-ref size for many rows holds what the few-row kernel needs of fewer,
+so that a workspace sized once leaves every call the kernel that it has in one of its own size."""
 import random
 
 import pytest
@@ -32,3 +33,20 @@ def test_size_covers_the_general_path(t, mode, monkeypatch):
             monkeypatch.setenv("TIERMM_QGEMM_TILE", "-")  # no plan: the general path's own
             assert both >= T.qgemm_ws_bytes(t, M, N, K, mode)
             monkeypatch.delenv("TIERMM_QGEMM_TILE")
+
+
+@pytest.mark.parametrize("mode", [T.MODE_F32, T.MODE_X3REF, "parts"], ids=["f32", "x3ref", "x3parts"])
+@pytest.mark.parametrize("t", TYPES)
+def test_size_covers_fewer_rows(t, mode, monkeypatch):
+    def size(M, N, K):
+        return T.qgemm_x3parts_ws_bytes(t, M, N, K) if mode == "parts" else T.qgemm_ws_bytes(t, M, N, K, mode)
+
+    for N, K in ((64, 256), (1024, 4096), (14336, 5120)):
+        for m in (1, 4, 5, 16, 17, 32, 33, 48):
+            own = size(m, N, K)
+            monkeypatch.setenv("TIERMM_QGEMM_TILE", "-")
+            general = size(m, N, K)
+            monkeypatch.delenv("TIERMM_QGEMM_TILE")
+            if own > general:  # the few-row kernel's need, or that of fewer rows still
+                for M in (m, 32, 48) if mode == T.MODE_F32 else (m, 32, 48, 49, 64, 300, 4096):
+                    assert M < m or size(M, N, K) >= own, (N, K, m, M)

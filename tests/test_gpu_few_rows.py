@@ -116,17 +116,44 @@ def test_few_rows_grouped(gpu, N, K):
 
 @pytest.mark.parametrize("mode", [T.MODE_F32, T.MODE_X3REF], ids=["f32", "x3ref"])
 @pytest.mark.parametrize("t,M,N,K", [(T.Q4_K, 16, 1024, 4096), (T.Q8_0, 3, 300, 1408)])
-def test_few_rows_in_a_workspace_of_the_general_path(gpu, t, M, N, K, mode):
-    """A workspace that an M of the general path was sized for: too small for the split sums of the
-    few-row kernel, which then leaves the call to the general path."""
+def test_few_rows_in_a_workspace_of_the_general_path(gpu, monkeypatch, t, M, N, K, mode):
+    """A workspace of the general path's own size: too small for the split sums of the few-row kernel,
+    which then leaves the call to the general path."""
+    monkeypatch.setenv("TIERMM_QGEMM_TILE", "-")
+    general = T.qgemm_ws_bytes(t, M, N, K, mode)
+    monkeypatch.delenv("TIERMM_QGEMM_TILE")
+    assert general < T.qgemm_ws_bytes(t, M, N, K, mode)
     blocks, w = _weight(t, N, K, 3, oracle.OUT_F32 if mode == T.MODE_F32 else oracle.OUT_F16)
     x = activations(M, K, seed=4)
     W, X, Y = hip.to_device(blocks), hip.to_device(x), hip.DeviceBuffer(M * N * 4)
-    for size in (T.qgemm_ws_bytes(t, 64, N, K, mode), T.qgemm_ws_bytes(t, M, N, K, mode)):
+    for size in (general, T.qgemm_ws_bytes(t, M, N, K, mode)):
         ws = hip.DeviceBuffer(size)
         T.qgemm(W.ptr, t, T.q_row_bytes(t, K), X.ptr, Y.ptr, M, N, K, mode=mode, ws=ws.ptr, ws_bytes=size)
         hip.synchronize()
         assert _err(Y.download(np.float32, M * N).reshape(M, N), x.astype(np.float64) @ w.T, x, w) <= BAR
+
+
+@pytest.mark.parametrize("t,M,N,K", [(T.Q4_K, 16, 1024, 4096), (T.Q5_0, 3, 300, 1408), (T.Q6_K, 32, 600, 2048)])
+def test_few_rows_parts_bits_in_workspaces_of_a_larger_batch(gpu, t, M, N, K):
+    """x3-ref, workspaces sized once for 512 rows: tiermm_qgemm and tiermm_qgemm_x3parts take the same
+    kernel for fewer rows, as in workspaces of their own sizes, and give the same bits."""
+    blocks, w = _weight(t, N, K, 5, oracle.OUT_F16)
+    x = activations(M, K, seed=6)
+    rb = T.q_row_bytes(t, K)
+    W, X, Y, P = hip.to_device(blocks), hip.to_device(x), hip.DeviceBuffer(M * N * 4), hip.DeviceBuffer(3 * M * K * 2)
+    T.split3(X.ptr, P.ptr, M * K, M * K, T.HML)
+    got = []
+    for rows in (M, 512):
+        a, b = T.qgemm_ws_bytes(t, rows, N, K), T.qgemm_x3parts_ws_bytes(t, rows, N, K)
+        ws = hip.DeviceBuffer(max(a, b))
+        T.qgemm(W.ptr, t, rb, X.ptr, Y.ptr, M, N, K, ws=ws.ptr, ws_bytes=a)
+        hip.synchronize()
+        got.append(Y.download(np.uint32, M * N))
+        T.qgemm_x3parts(W.ptr, t, rb, P.ptr, M * K, Y.ptr, M, N, K, ws=ws.ptr, ws_bytes=b, layout=T.PARTS_ROWS)
+        hip.synchronize()
+        got.append(Y.download(np.uint32, M * N))
+    assert _err(got[0].view(np.float32).reshape(M, N), x.astype(np.float64) @ w.T, x, w) <= BAR
+    assert all(np.array_equal(g, got[0]) for g in got[1:])
 
 
 @pytest.mark.parametrize("types,sizes,N,K", [

@@ -1017,6 +1017,16 @@ bool few_rows(int qt, int M, int N, int K, bool f32) {
 size_t few_rows_ws_bytes(int qt, int M, int N, int K, bool f32) {
   return few_rows(qt, M, N, K, f32) ? qgemm_skinny_ws_bytes(qt, M, N, K, f32, cus_or_default()) : 0;
 }
+// The most that the few-row kernel needs of a product of up to M rows.  The x-ref size queries return
+// no less, so that a workspace sized once for the largest batch takes every smaller one to the same
+// kernel, and tiermm_qgemm and tiermm_qgemm_x3parts, each with its own such workspace, to the same
+// bits.  F32 does so up to 48 rows; above, its general path's size alone is returned.
+size_t few_rows_ws_upto(int qt, int M, int N, int K, bool f32) {
+  size_t need = 0;
+  if (!f32 || M <= 48)
+    for (int m : {16, 32, 48}) need = std::max(need, few_rows_ws_bytes(qt, std::min(M, m), N, K, f32));
+  return need;
+}
 // The routed experts of type qt (weights, first rows, row counts), and whether all have few rows.
 struct TypeGroups {
   std::vector<const void*> W;
@@ -1531,7 +1541,7 @@ static size_t qgemm_general_ws_bytes(int qtype, int M, int N, int K, int mode) {
   return (size_t)N * K * sizeof(uint16_t) + parts;                   // W16 staged in the workspace
 }
 size_t tiermm_qgemm_ws_bytes(int qtype, int M, int N, int K, int mode) {
-  const size_t few = K % BK ? 0 : few_rows_ws_bytes(qtype, M, N, K, mode == TIERMM_MODE_F32);
+  const size_t few = K % BK ? 0 : few_rows_ws_upto(qtype, M, N, K, mode == TIERMM_MODE_F32);
   return std::max(few, qgemm_general_ws_bytes(qtype, M, N, K, mode));
 }
 
@@ -1653,7 +1663,7 @@ static size_t x3parts_general_ws_bytes(int qtype, int M, int N, int K) {
 }
 size_t tiermm_qgemm_x3parts_ws_bytes(int qtype, int M, int N, int K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % BK) return 0;
-  return std::max(few_rows_ws_bytes(qtype, M, N, K, false), x3parts_general_ws_bytes(qtype, M, N, K));
+  return std::max(few_rows_ws_upto(qtype, M, N, K, false), x3parts_general_ws_bytes(qtype, M, N, K));
 }
 
 int tiermm_qgemm_x3parts(const void* W, int qtype, size_t rb, const uint16_t* xparts, size_t part_stride,
