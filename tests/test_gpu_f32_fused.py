@@ -87,7 +87,7 @@ def test_f32_unfused_chunks(gpu):
     """K beyond the fused fp32 kernels (q4_K, K = 32768) and a type they do not decode
     (q4_0): fp32 rows expanded 960 at a time (256 MiB of expansion), three chunks with
     the last one partial, written at their column offsets of Y."""
-    M, K = 40, 32768
+    M, K = 56, 32768  # (more rows than the few-row kernel takes)
     for t, N in ((tier_amd.Q4_K, 2000), (tier_amd.Q4_0, 2000)):
         assert tier_amd.qgemm_plan(t, M, N, K) is None or t == tier_amd.Q4_K
         ws = tier_amd.qgemm_ws_bytes(t, M, N, K, tier_amd.MODE_F32)

@@ -93,8 +93,8 @@ def test_few_rows_nonfinite_scale(gpu):
 
 @pytest.mark.parametrize("N,K", [(1408, 512), (130, 1408)])
 def test_few_rows_grouped(gpu, N, K):
-    """70 experts (more than one launch holds) of 0 to 40 rows and of alternating types, more tiles
-    than the CUs: every expert's rows equal its own product."""
+    """70 experts of 0 to 31 rows and of three alternating types: one launch a type and number of
+    row tiles, some of them with more tiles than the CUs."""
     E = 70
     types = [T.Q8_0, T.Q5_0, T.Q8_0] if K % 256 else [T.Q4_K, T.Q5_0, T.Q6_K]
     rng = np.random.default_rng(N)
@@ -233,3 +233,41 @@ def test_few_rows_nonfinite_kq_scales(gpu, t):
     bad = np.isin(np.arange(N), rows)
     assert np.all(np.isnan(y[:, bad]))
     assert oracle.rel_fro(y[:, ~bad], (x.astype(np.float64) @ w.T)[:, ~bad]) <= BAR
+
+
+# experts of one type, rows of each, columns, K
+ROUTED = {
+    "packed, two launches": (T.Q4_K, [1 + i % 4 for i in range(70)], 192, 512),
+    "packed, many items": (T.Q4_K, [1 + i % 3 for i in range(64)], 1408, 512),
+    "packed, one unit": (T.Q6_K, [2] * 64, 1408, 256),
+    "packed, short unit": (T.Q5_0, [1 + i % 4 for i in range(68)], 640, 1408),
+    "packed and two tiles": (T.Q4_K, [1, 17, 4, 32, 2, 0, 25, 3, 31, 0, 18, 1], 300, 768),
+    "one tile, many items": (T.Q5_K, [5 + i % 12 for i in range(66)], 900, 512),
+    "one tile, short unit": (T.Q8_0, [1 + i % 16 for i in range(64)], 640, 1408),
+    "two tiles, many items": (T.Q4_K, [17 + i % 16 for i in range(40)], 1280, 512),
+    "two tiles, short unit": (T.Q5_0, [17 + i % 16 for i in range(40)], 1000, 1056),
+}
+
+
+@pytest.mark.parametrize("case", ROUTED)
+def test_few_rows_routed(gpu, case):
+    """Experts of one type each with its own weight (every 16 rows on in one matrix), each against
+    fp64: groups past the 64 of a launch, parts packed in a tile beside and without a second launch,
+    and more (expert, columns) items than the grid has workgroups (two a CU, one above 16 rows), so that
+    the ring of units runs on from one item into the next, with whole and short last units."""
+    t, sizes, N, K = ROUTED[case]
+    E, rb = len(sizes), T.q_row_bytes(t, K)
+    blocks, w = _weight(t, N + 16 * E, K, 41 + t, oracle.OUT_F16)
+    offs = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    P = int(offs[-1])
+    x = activations(P, K, seed=E)
+    W, X, Y = hip.to_device(blocks), hip.to_device(x), hip.DeviceBuffer(P * N * 4)
+    Y.fill_bytes(0xff)
+    T.qgemm_grouped([W.ptr + 16 * e * rb for e in range(E)], [t] * E, [rb] * E, X.ptr, offs, Y.ptr, N, K)
+    hip.synchronize()
+    got = Y.download(np.float32, P * N).reshape(P, N)
+    for e in range(E):
+        r = slice(offs[e], offs[e + 1])
+        if sizes[e]:
+            we = w[16 * e:16 * e + N]
+            assert _err(got[r], x[r].astype(np.float64) @ we.T, x[r], we) <= BAR, e

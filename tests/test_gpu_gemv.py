@@ -72,8 +72,8 @@ def test_gemv_ragged_shapes(gpu, t, N, K):
 @pytest.mark.parametrize("t", [tier_amd.Q8_0, tier_amd.Q4_0, tier_amd.Q4_1, tier_amd.Q5_0, tier_amd.Q5_1])
 @pytest.mark.parametrize("N,K", [(300, 14336), (9, 16384), (1029, 8192), (4100, 4096)])
 def test_gemv_block32_rows_in_lds(gpu, t, N, K):
-    """The 32-element block types staged whole in LDS: one row per wave above 80 KiB a
-    workgroup (K = 8192 .. 16384), two below; a partial last workgroup."""
+    """The 32-element block types on the dot kernel (q8_0 4100x4096: per-wave MFMA), x in up to
+    74 KiB of LDS: workgroups with one row more than others, and fewer rows than CUs."""
     rng = np.random.default_rng(N + K + t)
     be, _ = oracle.block(t)
     blocks = oracle.random_blocks(rng, t, N * (K // be)).reshape(N, -1)
@@ -141,10 +141,12 @@ def test_gemv_block32_unaligned_rows(gpu, t):
 
 
 @pytest.mark.parametrize("t", [tier_amd.Q5_K, tier_amd.Q8_0])
-@pytest.mark.parametrize("N,K", [(10250, 5120), (10256, 8192), (10240, 14336), (5000, 7936), (3000, 14336)])
+@pytest.mark.parametrize("N,K", [(10250, 5120), (10256, 8192), (10240, 14336), (5000, 7936), (3000, 14336),
+                                 (8185, 5120)])
 def test_gemv_mfma_tall(gpu, t, N, K):
-    """q5_K / q8_0 on the int8-MFMA kernel with more row tiles than CUs (eight waves a
-    workgroup) and ragged row counts, at each K class."""
+    """q5_K / q8_0 with more row tiles than CUs and ragged row counts, at each K class: q5_K on its
+    int8-MFMA kernels, q8_0 on its own at 8185x5120 (two tiles a workgroup) and 3000x14336, else on
+    the dot kernel."""
     rng = np.random.default_rng(N + K + t)
     be, _ = oracle.block(t)
     blocks = oracle.random_blocks(rng, t, N * (K // be)).reshape(N, -1)
@@ -190,8 +192,8 @@ def test_gemv_long_k_launch_shapes(gpu, t, N):
     """K = 14336 around the launch-shape boundaries: q4_K takes the whole-tile kernel from
     64 to 256 row tiles (1024 and 4096 rows), in split stages from 257 to 384 (4100,
     6144), two tiles a workgroup from 385 to 512 (6160, 8192), and the per-wave kernel
-    outside (1000, 8200); q5_K the same from 64 tiles; q8_0 switches at 256 tiles between
-    one tile x eight K parts and two tiles x four K parts per workgroup."""
+    above (8200); q5_K the same; below 64 tiles (1000) the dot kernel.  q8_0: the per-wave
+    kernel from 129 to 256 tiles (4096), one tile x eight K parts, the dot kernel outside."""
     K = 14336
     rng = np.random.default_rng(N + t)
     blocks = oracle.random_blocks(rng, t, N * (K // oracle.block(t)[0])).reshape(N, -1)
@@ -200,10 +202,12 @@ def test_gemv_long_k_launch_shapes(gpu, t, N):
     assert oracle.rel_fro(y, oracle.gemv_f64(blocks, t, x, N, K)) <= TOL
 
 
-@pytest.mark.parametrize("N,K", [(17, 256), (1000, 768), (4096, 4096), (4096, 5120), (4100, 5120)])
+@pytest.mark.parametrize("N,K", [(17, 256), (1000, 768), (4096, 4096), (4096, 5120), (4100, 5120), (4090, 256),
+                                 (4090, 768), (2060, 1280)])
 def test_gemv_q8_0_eight_k_parts(gpu, N, K):
-    """q8_0 at most 256 row tiles: one tile x eight K parts, down to K parts with no
-    group of eight blocks (K = 256, 768)."""
+    """q8_0 from 129 to 256 row tiles: one tile x eight K parts, down to K parts with no
+    group of eight blocks (K = 256, 768); 17 and 1000 rows on the dot kernel, 4100 on two tiles
+    a workgroup."""
     t = tier_amd.Q8_0
     blocks = quantized_weight(t, N, K, seed=N + K)
     x = activations(1, K, seed=K)[0]

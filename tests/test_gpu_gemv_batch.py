@@ -42,7 +42,7 @@ CASES = [
     ("q4_K four", tier_amd.Q4_K, (1024, 2048, 1040, 3000), 4096),  # ragged rows, K = 4096
     ("q4_K one", tier_amd.Q4_K, (1032,), 5120),
     ("q5_K two", tier_amd.Q5_K, (1024, 1024), 5120),
-    ("q4_K small (falls back)", tier_amd.Q4_K, (512, 4096), 5120),  # 32 tiles alone: per-wave kernel
+    ("q4_K small (falls back)", tier_amd.Q4_K, (512, 4096), 5120),  # 32 tiles alone: dot kernel
     ("q4_K long rows (falls back)", tier_amd.Q4_K, (2048, 1024), 14336),
     ("q6_K (falls back)", tier_amd.Q6_K, (1024, 1024), 5120),
     ("q8_0 (falls back)", tier_amd.Q8_0, (1024, 4096), 4096),

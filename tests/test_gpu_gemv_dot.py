@@ -1,7 +1,8 @@
 """The int8-dot decode GEMV (qgemv_dot.hip) at the edges of its shapes: one row, rows fewer and
 more than the CUs, units that do not fill the lanes of a row, rows of q3_K / q6_K that start
 two bytes off a dword, weights that start 4 bytes off a 16-byte boundary, K above the range of
-one pass over x, and block scales that are not finite.
+one pass over x, tall matrices (rows of 16, 32 and 64 lanes, odd and even counts of steps, several
+rows a slot, several parts a row), and block scales that are not finite.
 
 Bar: 2e-6 relative Frobenius against fp64.  Block sums are exact in int32 and rounded to
 fp32 once; a lane then adds at most K / (16 * 32) + 6 fp32 terms per row (34 at K = 14336,
@@ -16,7 +17,7 @@ from tier_amd import hip
 
 pytestmark = pytest.mark.gpu
 T = tier_amd
-# one shape per type that the dot kernel takes, chosen so that no other kernel does
+# shapes that no other kernel takes (but q5_K up to K = 5120, which its MFMA kernel does)
 SMALL = [T.Q4_0, T.Q4_1, T.Q5_0, T.Q5_1, T.IQ4_NL, T.Q8_0]
 SUPER = [T.Q2_K, T.Q3_K, T.IQ4_XS, T.Q4_K, T.Q5_K, T.Q6_K]
 SHAPES = [(1, 256), (3, 512), (255, 1280), (257, 2304), (600, 5376), (40, 14336), (17, 18432)]
@@ -71,6 +72,27 @@ def test_dot_gemv_nonfinite_scale(gpu, t):
     assert oracle.rel_fro(y[ok], oracle.gemv_f64(blocks, t, x, N, K)[ok]) <= 2e-6
 
 
+# units of 64 elements (iq4), of 128 (q2_K, q3_K) on 256 CUs: lanes a row, steps a row, rows a slot
+TALL = [(14336, 5120),  # 16, 5, 1; 16, 3, 1
+        (9001, 2304),   # 64, 1, 3; 32, 1, 2; ragged rows a workgroup, q3_K rows at both phases
+        (4097, 5376),   # 32, 3, 1; 64, 1, 2
+        (2500, 8192),   # 64, 2, 1; 64, 1, 1
+        (20001, 1024),  # 16, 1, 2
+        (5120, 14336)]  # 64, 1, 5 in four parts; 64, 1, 3 in two
+
+
+@pytest.mark.parametrize("N,K", TALL)
+@pytest.mark.parametrize("t", [T.IQ4_XS, T.IQ4_NL, T.Q2_K, T.Q3_K])
+def test_dot_gemv_tall(gpu, t, N, K):
+    """Every row: the largest error against the outputs' root mean square (34 roundings of sums up
+    to some four times that: 1e-5)."""
+    blocks, x = _blocks(t, N, K, N + K + t)
+    want = oracle.gemv_f64(blocks, t, x, N, K)
+    y = _run(blocks, t, x, N, K)
+    assert oracle.rel_fro(y, want) <= 2e-6
+    assert np.abs(y - want).max() <= 1e-5 * np.sqrt(np.mean(want ** 2))
+
+
 def _zero_at(t, b, j):
     """Element j < 16 of each 32-element block (of each 256-element one, for the K types) set to weight 0."""
     b = b.copy()
@@ -107,9 +129,10 @@ def _zero_at(t, b, j):
 @pytest.mark.parametrize("t", [T.Q4_0, T.Q4_1, T.Q5_0, T.Q5_1, T.Q8_0, T.Q2_K, T.Q3_K, T.Q6_K])
 def test_dot_gemv_outlier_in_x(gpu, t, mag):
     """An outlier of x where every row's weight is zero, beside ordinary values: its block's other
-    elements keep the bits that fp32 sums would give them.  Outliers in every block and in every third."""
+    elements keep the bits that fp32 sums would give them.  Outliers in every block and in every third;
+    rows in several parts, and several rows a slot (9001; q6_K's dot kernel stops short of that)."""
     be, bb = oracle.block(t)
-    for N, K, step in ((40, 1280, 1), (257, 14336, 3), (1000, 2304, 1)):
+    for N, K, step in ((40, 1280, 1), (257, 14336, 3), (1000 if t == T.Q6_K else 9001, 2304, 1)):
         blocks, x = _blocks(t, N, K, 5 * N + t)
         b = _zero_at(t, blocks.reshape(N, -1, bb), 5).reshape(N, -1)
         at = np.arange(5, K, be)[::step]

@@ -5,16 +5,17 @@ Non-finite x.  gemv_q sums q_val * x in fp32, so a NaN anywhere in x makes every
 y NaN, and +-Inf at column k makes row r +-Inf (sign of q_val(r, k) * x[k]) or
 NaN (q_val(r, k) == 0, or terms of both signs).  The int8-digit kernels carry
 finite x only and must still give that pattern; every kernel family is driven
-here (whole-tile q4_K/q5_K, per-wave q4_K/q5_K/q8_0, q6_K, the staged 32-element
-block kernel, the generic kernel).  Expected: the oracle's restatement of
+here (whole-tile q4_K/q5_K, per-wave q4_K/q5_K/q8_0, q6_K, the dot kernel, the
+generic kernel).  Expected: the oracle's restatement of
 gemv_q's own lane-order fp32 sum (orc_gemv_lanes), whose NaN / +Inf / -Inf
 pattern must match exactly; the fp64 closed form (orc_gemv_f64) must agree with
 it, which pins the pattern independently of the summation order.
 
 Long K.  The reference loop has no K bound.  q4_K, q5_K and q8_0 rows up to
 K = 28672 run on the int8-MFMA kernel (x digits of the whole row in 121 KiB of
-LDS); q6_K above 14336 and the other types above 16384 on the generic kernel,
-which reads x from global memory.  Bar: relative Frobenius error <= 1e-5 against
+LDS); what that kernel and q6_K's do not take on the dot kernel up to K = 36352
+(x in 160 KiB); longer rows and the other types on the generic kernel, which
+above 16384 reads x from global memory.  Bar: relative Frobenius error <= 1e-5 against
 fp64.
 """
 import numpy as np
@@ -49,23 +50,28 @@ KERNELS = [
     (tier_amd.Q4_K, 5120, 5120, "q4K-whole-tile-2-tiles"),
     (tier_amd.Q4_K, 1024, 14336, "q4K-whole-tile-k14336"),
     (tier_amd.Q4_K, 10240, 8192, "q4K-whole-tile-k8192"),
-    (tier_amd.Q4_K, 512, 5120, "q4K-per-wave-1x4"),
+    (tier_amd.Q4_K, 512, 5120, "q4K-dot"),
     (tier_amd.Q4_K, 5120, 14336, "q4K-whole-tile-split-stages"),
     (tier_amd.Q4_K, 8192, 14336, "q4K-whole-tile-k14336-2-tiles"),
     (tier_amd.Q4_K, 9000, 14336, "q4K-per-wave-2x4"),
-    (tier_amd.Q4_K, 512, 14336, "q4K-per-wave-1x8"),
+    (tier_amd.Q4_K, 512, 14336, "q4K-dot-k14336"),
+    (tier_amd.Q4_K, 5120, 7936, "q4K-per-wave-2x4-k8192"),
     (tier_amd.Q5_K, 13824, 5120, "q5K-whole-tile"),
     (tier_amd.Q5_K, 1024, 5120, "q5K-whole-tile-1-tile"),
     (tier_amd.Q5_K, 512, 5120, "q5K-per-wave"),
     (tier_amd.Q5_K, 5120, 14336, "q5K-whole-tile-split-stages"),
     (tier_amd.Q5_K, 4096, 14336, "q5K-whole-tile-k14336"),
+    (tier_amd.Q5_K, 1500, 7936, "q5K-per-wave-k8192"),
     (tier_amd.Q8_0, 4096, 4096, "q8_0-per-wave"),
-    (tier_amd.Q8_0, 10240, 8192, "q8_0-per-wave-tall"),
-    (tier_amd.Q6_K, 1024, 5120, "q6K"),
+    (tier_amd.Q8_0, 8000, 4096, "q8_0-per-wave-tall"),
+    (tier_amd.Q8_0, 10240, 8192, "q8_0-dot-tall"),
+    (tier_amd.Q6_K, 1024, 5120, "q6K-dot"),
+    (tier_amd.Q6_K, 2600, 5120, "q6K"),
     (tier_amd.Q6_K, 5120, 14336, "q6K-long"),
-    (tier_amd.Q4_0, 300, 4096, "q4_0-staged"),
-    (tier_amd.Q5_1, 300, 4096, "q5_1-staged-min"),
-    (tier_amd.Q2_K, 200, 1024, "q2K-generic"),
+    (tier_amd.Q4_0, 300, 4096, "q4_0-dot"),
+    (tier_amd.Q5_1, 300, 4096, "q5_1-dot-min"),
+    (tier_amd.Q2_K, 200, 1024, "q2K-dot"),
+    (tier_amd.IQ3_XXS, 200, 1024, "iq3_xxs-generic"),
 ]
 
 
