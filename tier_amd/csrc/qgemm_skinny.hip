@@ -60,12 +60,13 @@ constexpr int SK_UNIT = 256;      // K per step of the K loop (8 MFMA steps of 3
 
 struct SkArgs {
   const uint16_t* X;  // fragments [unit][step 8][part][tile][64 lanes][8 halfs]
-  const uint16_t* S;  // F32, formats with minima: sub-block sums [unit][tile][t 2][64 lanes][4 halfs]
+  const uint16_t* S;  // F32, formats with minima: sub-block sums [unit][tile][t 2][64 lanes][4 halfs], or with
+                      // one row tile a group (flat) [unit][tile][sub-block 8][16 rows] floats
   float* Y;
   float* P;           // KS > 1: partial sums of split z at P + z * ps, rows of N floats
   const int32_t* xexp;
   size_t rb, ps;
-  int ldy, N, K, KS, mtot, ngroups;
+  int ldy, N, K, KS, mtot, ngroups, flat;
   float beta;
   int tile0[SK_G + 1];  // workgroup tiles of group g: [tile0[g], tile0[g + 1])
   int row0[SK_G], rows[SK_G], mt0[SK_G];  // rows of x and Y; its first x tile
@@ -169,8 +170,8 @@ __global__ __launch_bounds__(1024) void sk_relayout3(const uint16_t* __restrict_
 
 // F32: the two-part split with a power of two per row (x3s_split's), and with S the
 // sub-block sums S_b = sum of hi + lo (what the products see of x) over the 32 elements of
-// sub-block b, over 32, in two fp16 parts: lane (m, kg) of the unit's sum fragment t holds
-// hi, hi, lo, lo of sub-block b = 4 (kg % 2) + 2 (kg / 2) + t.
+// sub-block b: fp32 values (flat), or over 32 in two fp16 parts: lane (m, kg) of the unit's sum
+// fragment t holds hi, hi, lo, lo of sub-block b = 4 (kg % 2) + 2 (kg / 2) + t.
 template <bool PACK>
 __global__ __launch_bounds__(1024) void sk_split2(const float* __restrict__ x, const SkArgs p, uint16_t* __restrict__ X,
                                                  uint16_t* __restrict__ S, int32_t* __restrict__ xexp) {
@@ -212,11 +213,15 @@ __global__ __launch_bounds__(1024) void sk_split2(const float* __restrict__ x, c
       float sum = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
       sum += __shfl_xor(sum, 1, 64);
       sum += __shfl_xor(sum, 2, 64);
-      sum *= 0.03125f;
-      const uint32_t s0 = f2h(sum), s1 = f2h(sum - h2f((uint16_t)s0));
+      const float s32 = sum * 0.03125f;
+      const uint32_t s0 = f2h(s32), s1 = f2h(s32 - h2f((uint16_t)s0));
       const int b = (k >> 5) & 7, kg = 2 * ((b >> 1) & 1) + (b >> 2);
       uint16_t* f = S + ((size_t)(k >> 8) * p.mtot + tile) * 512;
-      if ((k & 31) == 0) {
+      if ((k & 31) == 0 && p.flat) {
+        float* o = (float*)f + 16 * b + m;
+        *o = sum;
+        if (PACK) o[sk_pack(true)] = 0.f;
+      } else if ((k & 31) == 0) {
         u32x2* o = (u32x2*)(f + 256 * (b & 1) + (16 * kg + m) * 4);
         *o = u32x2{s0 * 0x10001u, s1 * 0x10001u};
         if (PACK) o[sk_pack(true)] = u32x2{0, 0};  // the sums count once, with the hi parts
@@ -297,18 +302,21 @@ __device__ __forceinline__ uint32_t kq_bytes(u32x4 h, int kh) {
   const uint32_t lo = MIN ? h[2] : h[1];
   return kh ? ((h[3] >> (MIN ? 4 : 0)) & 0x0f0f0f0fu) | ((lo >> 2) & 0x30303030u) : lo & 0x3f3f3f3fu;
 }
-// q4_K / q5_K, codes centred by C: the factor C d sc - dmin m of this lane's sub-block in two fp16
-// parts, times a power of two that keeps it below 2^15 (126 max(C |d|, |dmin|) bounds it), against
-// the hi and lo sums, in the lanes kg % 2 == kh and zero in the others; inv = 32 over that power,
-// which takes the product to the factor's own scale
+// q4_K / q5_K, codes centred by C: the factor C d sc - dmin m of this lane's sub-block
+template <int C>
+__device__ __forceinline__ float kq_factor(u32x4 h, int kh, int t, int kg) {
+  const int sh = 16 * (kg >> 1) + 8 * t;
+  const float m = h2f(h[0] >> 16) * (float)((kq_bytes<true>(h, kh) >> sh) & 0xffu);  // exact
+  return fmaf((float)C * h2f(h[0] & 0xffffu), (float)((kq_bytes<false>(h, kh) >> sh) & 0xffu), -m);
+}
+// The same in two fp16 parts, times a power of two that keeps it below 2^15 (126 max(C |d|, |dmin|)
+// bounds it), against the hi and lo sums, in the lanes kg % 2 == kh and zero in the others; inv = 32
+// over that power, which takes the product to the factor's own scale
 template <int C>
 __device__ __forceinline__ u32x2 kq_offset(u32x4 h, int kh, int t, int kg, float& inv) {
-  const int sh = 16 * (kg >> 1) + 8 * t;
-  const float cd = (float)C * h2f(h[0] & 0xffffu), dm = h2f(h[0] >> 16);
-  const float m = dm * (float)((kq_bytes<true>(h, kh) >> sh) & 0xffu);  // exact
-  const float b = fmaf(cd, (float)((kq_bytes<false>(h, kh) >> sh) & 0xffu), -m);
+  const float b = kq_factor<C>(h, kh, t, kg);
   // the exponent is 0 for 0, Inf and NaN; non-finite factors stay so
-  const int e = 8 - __builtin_amdgcn_frexp_expf(fmaxf(fabsf(cd), fabsf(dm)));
+  const int e = 8 - __builtin_amdgcn_frexp_expf(fmaxf((float)C * fabsf(h2f(h[0] & 0xffffu)), fabsf(h2f(h[0] >> 16))));
   inv = ldexpf(32.f, -e);
   const float v = ldexpf(b, e);
   const uint32_t hi = f2h(v), lo = f2h(v - h2f((uint16_t)hi));
@@ -345,11 +353,12 @@ struct Sk<QT_Q4_K> {
     }
   }
   __device__ __forceinline__ float norm() const { return 1.f; }
-  // (a d that is not finite makes the offset's parts, and the row, NaN)
+  // (a d that is not finite makes the factor or its parts, and the row, NaN)
   __device__ __forceinline__ float post(float) const { return h2f(h[0] & 0xffffu) * 0x1p14f; }
   __device__ __forceinline__ u32x2 offset(int kh, int t, int kg, float& inv) const {
     return kq_offset<8>(h, kh, t, kg, inv);
   }
+  __device__ __forceinline__ float factor(int kh, int t, int kg) const { return kq_factor<8>(h, kh, t, kg); }
 };
 
 template <>
@@ -384,11 +393,12 @@ struct Sk<QT_Q5_K> {
     }
   }
   __device__ __forceinline__ float norm() const { return 1.f; }
-  // (a d that is not finite makes the offset's parts, and the row, NaN)
+  // (a d that is not finite makes the factor or its parts, and the row, NaN)
   __device__ __forceinline__ float post(float) const { return h2f(h[0] & 0xffffu) * 0x1p14f; }
   __device__ __forceinline__ u32x2 offset(int kh, int t, int kg, float& inv) const {
     return kq_offset<16>(h, kh, t, kg, inv);
   }
+  __device__ __forceinline__ float factor(int kh, int t, int kg) const { return kq_factor<16>(h, kh, t, kg); }
 };
 
 template <>
@@ -728,7 +738,21 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
         for (int i = 0; i < WR; ++i) {
           float s = cur[i].post(nm[i]);
           if constexpr (!L::MINS) asm volatile("" : "+v"(s));  // (else the NaN select moves behind each product)
-          if constexpr (L::MINS) {
+          if constexpr (L::MINS && MT == 1) {
+            // one row tile: 8 fp32 products take fewer instructions than the factor's two parts, which
+            // cost as much for one tile as for three (q4_K 14336x5120, us: M = 2 27.0 -> 25.9, M = 16
+            // 29.6 -> 27.3)
+            const uint32_t b = __float_as_uint(cur[i].factor(kh, t, kg));
+            const auto bb = __builtin_amdgcn_permlane32_swap(b, b, false, false);  // sub-blocks 4 kh + t, 4 kh + 2 + t
+            const float* sp = (const float*)(xs - lane * 16 + 8 * NP * 1024) + 16 * (4 * kh + t) + 4 * kg;
+            const float4v s0 = *(const float4v*)sp, s1 = *(const float4v*)(sp + 32);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              acc[i][0][r] = fmaf(s0[r], __uint_as_float(bb[0]), acc[i][0][r]);
+              acc[i][0][r] = fmaf(s1[r], __uint_as_float(bb[1]), acc[i][0][r]);
+              acc[i][0][r] = fmaf(c[i][0][r], s, acc[i][0][r]);
+            }
+          } else if constexpr (L::MINS) {
             float inv;
             const half4 off = __builtin_bit_cast(half4, cur[i].offset(kh, t, kg, inv));
 #pragma unroll
@@ -918,7 +942,7 @@ int qgemm_skinny(const void* const* W, int qt, const int* row0, const int* rows,
     const bool pack = kind == 0;
     const int mt = std::max(kind, 1);
     SkArgs a{};
-    a.Y = Y; a.rb = rb; a.ldy = ldy; a.N = N; a.K = K; a.KS = ks; a.beta = beta;
+    a.Y = Y; a.rb = rb; a.ldy = ldy; a.N = N; a.K = K; a.KS = ks; a.beta = beta; a.flat = mt == 1;
     int total = 0, last = 0;
     for (; g0 < n && a.ngroups < SK_G; ++g0) {
       if ((packed && rows[g0] <= 16 ? 0 : (rows[g0] + 15) / 16) != kind) continue;
