@@ -7,9 +7,8 @@
 // block scales for the row exponents) and multiplies 128- or 256-row tiles that are mostly
 // padding.  Here a lane decodes the 16 weights that it holds as an MFMA operand, in registers:
 //   - the bytes of a unit (256 elements of 16 * WR * RW rows) come by LDS DMA, whose consecutive
-//     lanes read consecutive 16-byte chunks of a row.  Loaded straight into the lanes that need
-//     them, 16 rows apart, each load took 64 cycles of the CU's return path, which was then busy
-//     70 % of the time;
+//     lanes read consecutive 16-byte chunks of a row (loaded straight into the lanes that need
+//     them, every lane of a load is in another row);
 //   - codes are read as fp16 subnormals (no conversions), and for F32 the block scale is applied
 //     to the sums where the code times its sub-block scale is a whole number that fp16 holds
 //     (q4_K, q5_K: two products, x hi and lo, where the fused kernel has three, and no pass over
@@ -19,15 +18,16 @@
 //     difference, and what rounds in either stays: q4_K 300x5120, M = 37, rows of x that are
 //     constant 1.1e-5 off 64 bits -> 2.8e-7, 3 + n 1.2e-6 -> 2.1e-7 (fused kernel 4.0e-7);
 //   - x is split and laid out as operand fragments once, by a launch before.
-// Measured, all launches of a call, in us (fused kernel -> this one):
-//   F32, N = 14336, K = 5120:  q4_K M = 2  59.7 -> 24.5, M = 37  62.7 -> 39.5;
-//     q6_K M = 2  61.0 -> 32.5, M = 37  65.1 -> 46.0;  q8_0 M = 2  69.1 -> 31.4
-//   F32, N = 1024, K = 4096:  q4_K M = 2  22.9 -> 14.0
-//   x-ref, N = 14336, K = 5120 (before the parts were packed):  q4_K M = 2  44.9 -> 27.7, M = 32  43.0 -> 32.5;
-//     q6_K M = 16  54.1 -> 34.6;  q8_0 M = 16  62.6 -> 41.5
-// with errors against fp64 no larger (F32 q4_K, N(0, 1): 4.0e-7 -> 1.4e-7).  What
-// is left over the weights' read (8 us at q4_K) is the split and reduce launches (9 us), the
-// first unit's latency and, per unit, decode, MFMAs and LDS reads that overlap in part.
+// Measured, all launches of a call, in us, graph replays over rotated weights (fused kernel -> this one):
+//   F32, N = 14336, K = 5120:  q4_K M = 2  58.7 -> 25.9, M = 37  61.3 -> 39.2;  q5_K M = 2  63.5 -> 28.7,
+//     M = 37  66.0 -> 41.9;  q6_K M = 2  61.6 -> 34.6, M = 37  64.2 -> 47.3;  q8_0 M = 2  69.9 -> 32.6
+//   F32, N = 1024, K = 4096:  q4_K M = 2  23.8 -> 14.3, M = 37  25.3 -> 21.0
+//   x-ref, N = 14336, K = 5120:  q4_K M = 2  45.8 -> 24.3, M = 16  47.9 -> 27.3, M = 32  44.3 -> 31.7;
+//     q6_K M = 16  56.9 -> 34.9;  q8_0 M = 16  63.6 -> 38.5;  q5_0 M = 4  49.6 -> 29.0
+// with errors against fp64 no larger (F32 q4_K, N(0, 1): 4.0e-7 -> 1.4e-7).  What is left over the
+// weights' read (8 us at q4_K) is the split and reduce launches (4 to 5 us each) and, at M = 37 in the
+// kernel's 34 us, 15 us of VALU issue (mostly decode), 7 of MFMAs, 6 of LDS reads and 13 of the
+// vector memory's return path, which overlap in part: four waves a SIMD meet at a barrier every unit.
 #include <algorithm>
 
 #include "tm_device.h"
@@ -50,8 +50,9 @@ constexpr int SK_WR = 2;          // 16-row W tiles of a wave
 // (x-ref three parts of 4 rows, F32 two of 8).  One product then does the work of three (two), x takes
 // a third (half) of the loads and LDS, and that room holds a third unit of weights in flight and the
 // meeting apart from the ring, so the loads no longer stop between two items.
-// Measured, us a call: 8 tokens, top 8 of 64 experts, hidden 2048, ffn 1408 (both products and the
-// combine) 127 -> 108, 1 token 44.7 -> 41.9; F32 q4_K 14336x5120 M = 8 27.1 -> 26.2.
+// Measured before and after on one card, us a call: 8 tokens, top 8 of 64 experts, hidden 2048, ffn
+// 1408 (both products and the combine) 127 -> 108, 1 token 44.7 -> 41.9; F32 q4_K 14336x5120 M = 8
+// 27.1 -> 26.2.  (The fused kernel took 243 for the 8 tokens.)
 constexpr int sk_pack(bool f32) { return f32 ? 8 : 4; }
 // Row waves of a workgroup, each for four K quarters, by the row tiles of x
 constexpr int sk_rw(int mt) { return mt == 1 ? 2 : 4; }
@@ -618,7 +619,8 @@ __global__ __launch_bounds__(256 * sk_rw(MT))
         }
       }
       if (D::TAIL && wave >= TW) {
-        // the dword after the chunks, where a byte of the unit lies in it
+        // the dword after the chunks, where a byte of the unit lies in it (where W's last row ends in the
+        // middle of a dword, the rest of that dword is read too)
         const int off = D::UB % 16 || (tsrc & 2) ? 16 * CH : 16 * CH - 4;
         dma4((const void*)((tsrc & ~(uintptr_t)3) + off), base + L::WG * 1024 + (uint32_t)(wave - TW) * 256);
         tsrc += D::UB;
@@ -880,7 +882,7 @@ int sk_splits(int mt, int N, int K, int cus) {
 // Whether the few-row kernel takes an M-row product (or an expert of M rows) of this type: up to
 // the row tiles whose fragments fit in LDS beside the weights (F32: 48 rows, q8_0 32; x-ref: 32,
 // q8_0 16).  It is the faster one up to there at every shape measured, least at its largest M of
-// a small weight (N = 1024, K = 4096: q4_K F32 M = 48 24.5 -> 21.0 us, x-ref M = 32 20.1 -> 18.9);
+// a small weight (N = 1024, K = 4096: q4_K F32 M = 48 25.5 -> 21.9 us, x-ref M = 32 19.5 -> 18.3);
 // a variant with a fourth row tile (one wave set a CU, spills) lost at M = 64, 61.6 -> 70.7 us.
 bool qgemm_skinny_takes(int qt, int M, int N, int K, bool f32) {
   return M >= 1 && N >= 1 && K >= 1 && M <= 16 * (f32 ? sk_max_tiles<true>(qt) : sk_max_tiles<false>(qt));

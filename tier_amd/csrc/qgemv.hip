@@ -204,23 +204,23 @@ int qgemv_dispatch(const void* W, int qtype, size_t rb, const float* x, float* y
     case QT_F32: return launch_dense<TIERMM_F32>(W, x, y, N, K, s);
     case QT_F16: return launch_dense<TIERMM_F16>(W, x, y, N, K, s);
     case QT_BF16: return launch_dense<TIERMM_BF16>(W, x, y, N, K, s);
-    case QT_Q4_K:  // below 64 row tiles the dot kernel: 301x8192 8.6 -> 4.6 us, 640x5120 5.2 -> 4.4
+    case QT_Q4_K:  // below 64 row tiles the dot kernel: 301x8192 8.6 -> 4.6 us, 640x5120 5.25 -> 4.6
       if (qgemv_ws_takes(QT_Q4_K, N, K)) return qgemv_q4k_ws(W, rb, x, y, N, K, s);
       if (tiles >= 64 && K <= kQ4kMaxK) return qgemv_q4k(W, rb, x, y, N, K, s);
       break;
-    case QT_Q5_K:  // the same above K = 5120 (301x8192 9.5 -> 6.2 us; 640x5120 5.65 against 6.1)
+    case QT_Q5_K:  // the same above K = 5120 (301x8192 9.6 -> 6.6 us; 640x5120 5.7 against 6.5)
       if (qgemv_mfma_fits(W, qtype, rb, K) && (tiles >= 64 || K <= 5120))
         return qgemv_ws_takes(QT_Q5_K, N, K) ? qgemv_q5k_ws(W, rb, x, y, N, K, s) : qgemv_mfma(W, qtype, rb, x, y, N, K, s);
       break;
     case QT_Q8_0:
-      // MFMA where it measured faster: 129-512 row tiles up to K = 5120 (4096x5120 6.2 against
-      // 7.9 us; 1024x5120 5.45 against 4.75, 20000x5120 27.7 against 22.6), 129-256 above 8192
-      // (4096x14336 12.9 against 14.6; 5120x14336 18.0 against 17.2); not between (2500x8192
-      // 12.1 against 7.6)
+      // MFMA where it measured faster: 129-512 row tiles up to K = 5120 (4096x5120 6.7 against
+      // 8.3 us, 8192x5120 11.0 against 11.4; 1024x5120 5.3 against 4.8, 20000x5120 29.2 against
+      // 22.3), 129-256 above 8192 (4096x14336 14.2 against 15.1; 5120x14336 20.4 against 18.2); not
+      // between (2500x8192 11.8 against 7.9)
       if (qgemv_mfma_fits(W, qtype, rb, K) && tiles > 128 && (K <= 5120 ? tiles <= 512 : K > 8192 && tiles <= 256))
         return qgemv_mfma(W, qtype, rb, x, y, N, K, s);
       break;
-    case QT_Q6_K:  // MFMA above 160 row tiles (4096x5120 7.9 against 8.6 us; 2500x4096 7.1 against 6.6)
+    case QT_Q6_K:  // MFMA above 160 row tiles (4096x5120 7.9 against 9.8 us; 2500x4096 7.1 against 6.7)
       if (tiles > 160 && qgemv_q6k_fits(W, rb, N, K)) return qgemv_q6k(W, rb, x, y, N, K, s);
       break;
     default: break;

@@ -22,15 +22,19 @@
 // the slots (1024 / L per workgroup) come out even.  The next unit's bytes are loaded
 // before the current one is computed, and the first before x is prepared.
 //
-// Measured (MI355X, us per call over rotated copies; before: the generic or staged kernel for
-// the first four, MFMA for the rest).  At 14336x5120 the loop is VALU-bound: 3.0 (q4_0) to
-// 5.3 (iq4_xs) instructions per weight where the weight bytes alone would take 7 us.
-//   iq4_xs 14336x5120 49.5 -> 15.3, 5120x14336 97 -> 17.8, 1024x5120 14.3 -> 4.6
-//   q3_K   14336x5120 35.6 -> 17.1, 4096x14336 52.7 -> 15.4, 1024x5120 13.4 -> 4.9
-//   q2_K   14336x5120 20.6 -> 16.4, 5120x14336 62 -> 16.9
-//   q4_0   14336x5120 22.7 -> 12.0, 5120x14336 37 -> 14.7, 4096x14336 29.8 -> 11.8
-//   q8_0   9000x8192 23.2 -> 16.5, 20000x5120 27.7 -> 22.6, 1024x5120 5.45 -> 4.75
-//   q6_K   1024x5120 7.6 -> 5.0, 2500x8192 14.0 -> 9.1, 9001x11264 49.4 -> 26.7
+// Measured (MI355X, us a call, graph replays over rotated copies of the weight; before: the generic
+// kernel for iq4 and the K types, one that staged rows in LDS for q4 and q5, MFMA for the others):
+//   iq4_xs 14336x5120 54.4 -> 14.5, 5120x14336 113 -> 17.0, 1024x5120 14.9 -> 4.9;  iq4_nl 53.4 -> 13.7
+//   q3_K   14336x5120 39.1 -> 17.2, 4096x14336 67 -> 16.4, 1024x5120 15.6 -> 4.9
+//   q2_K   14336x5120 27.1 -> 15.9, 5120x14336 85 -> 17.3
+//   q4_0   14336x5120 22.3 -> 11.4, 5120x14336 36.0 -> 13.6, 4096x14336 29.2 -> 11.4
+//   q4_1, q5_0, q5_1 14336x5120 21.4 -> 11.7, 27.2 -> 13.2, 27.6 -> 13.7
+//   q8_0   9000x8192 24.5 -> 17.6, 20000x5120 29.2 -> 22.3, 1024x5120 5.3 -> 4.8
+//   q6_K   1024x5120 7.7 -> 5.4, 2500x8192 14.0 -> 10.5, 9001x11264 69 -> 29.2
+// What bounds it at 14336x5120 (counters): 2.6 (q4_0) to 4.8 (q3_K) VALU instructions a weight,
+// x included, whose issue takes 4.8 to 9.0 us a SIMD; LDS reads of x that take 4.5 us a CU (units of
+// 128: 9, two thirds of it bank conflicts of lanes four blocks apart); the weight's bytes at a large
+// copy's rate 8.5 us (q4_0), in part overlapped, after some 3 us of launch, x and first loads.
 // Two rows a lane, 512-thread workgroups (one or two per CU) and deeper prefetch were within
 // 10 % of this on large shapes and slower on small ones.
 //
@@ -58,10 +62,8 @@ namespace {
 
 constexpr int XB = 36;  // dwords of a prepared 32-element block of x
 
-// Register loads start at dword boundaries: on gfx950 a 16-byte load at a 4-byte aligned
-// address costs 17 cycles of the vector cache for lanes up to 36 bytes apart (33 at 108
-// bytes), one at a 2-byte aligned address 65 (96 at 110 bytes).  Bytes that start two past a
-// dword are shifted into place with v_alignbit.
+// Register loads start at dword boundaries (the vector cache splits those that do not into more
+// accesses); bytes that start two past a dword are shifted into place with v_alignbit.
 typedef uint32_t u32x4d __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u32x2d __attribute__((ext_vector_type(2), aligned(4)));
 #define TM_GLOBAL __attribute__((address_space(1)))

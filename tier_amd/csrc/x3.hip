@@ -1093,10 +1093,12 @@ int big_group_chunk(const int* offs, int n_experts, int N, int K) {
 // Products below the big-tile kernel: 128 x 128 tiles where they come near filling the 256 CUs, else
 // 64 x 64 ones, four times as many (each output is summed in the same order: the same bits).  With
 // two workgroups or more on a CU the loads of one cover the other's products, which one 128-tile
-// workgroup on some of the CUs cannot.  Whole calls on f16 rows, 128 -> 64 tiles, us: 5120x4096
-// M = 2 110 -> 59, M = 203 (80 tiles) 114 -> 73, M = 512 (160 tiles) 118 -> 109; 5120x14336 M = 512
-// 558 -> 437; 1024x5120 M = 512 149 -> 88.  At 224 tiles the 128-wide ones win: 14336x5120 M = 203
-// 166, 64-wide 202.
+// workgroup on some of the CUs cannot.  Whole calls on f16 rows, rotated weights, 128 -> 64 tiles, us:
+// 5120x4096 M = 2 115 -> 76, M = 203 (80 tiles) 122 -> 86, M = 512 (160 tiles) 128 -> 121; 5120x14336
+// M = 512 522 -> 444; 1024x5120 M = 512 149 -> 89.  At 224 tiles the 128-wide ones win: 14336x5120
+// M = 203 166, 64-wide 202 (one weight, in the caches); nothing between 160 and 224 was measured.
+// What is left is the serial walk over K: M = 2 of 5120x14336 takes 263 us, and the 64-tile kernel's
+// return path of loads is busy 55 of its 83 us at M = 203.
 template <int MODE>
 int launch_x3_small(const X3Args& a, hipStream_t s, const char* who) {
   const long tiles = (long)((a.M + 127) / 128) * ((a.N + 127) / 128);
