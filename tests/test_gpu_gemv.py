@@ -338,3 +338,15 @@ def test_gemv_split_stages(gpu, t, N, K):
         assert np.array_equal(r.view(np.uint32), y.view(np.uint32))
     oy = OY.download(np.float32, 5120)
     assert oracle.rel_fro(oy, oracle.gemv_f64(o_blocks, tier_amd.Q4_K, o_x, 5120, 14336)) <= TOL
+
+
+@pytest.mark.parametrize("t", [tier_amd.Q4_K, tier_amd.Q5_K])
+@pytest.mark.parametrize("N,K", [(1024, 5120), (40, 5120), (300, 16384), (4112, 14336), (1024, 8192)])
+def test_gemv_constant_and_two_valued_x(gpu, t, N, K):
+    """x of one or two values: what rounds in a sub-block's sum of x is then the same everywhere, and
+    may not add up over the row (one step of 2^-24 in each of the minima's terms, which are some 180
+    times the result, would be 1.1e-5)."""
+    blocks = quantized_weight(t, N, K, seed=N + t)
+    n = activations(1, K, seed=K)[0]
+    for x in (np.full(K, 0.1, np.float32), np.where(n > 0, 0.1, 0.3).astype(np.float32)):
+        assert oracle.rel_fro(_gemv(blocks, t, x, N, K), oracle.gemv_f64(blocks, t, x, N, K)) <= 5e-6

@@ -48,12 +48,15 @@ __device__ __forceinline__ bool flags_any(const int* flags, int n) {
 template <bool DSUM = false>
 __device__ __forceinline__ void prep_half(int s, int h, const float (&v)[16], uint8_t* xq, float* meta,
                                           int* dsum = nullptr) {
-  float amax = 0.f, sum = 0.f;
+  float amax = 0.f;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    amax = fmaxf(amax, fabsf(v[i]));
-    sum += v[i];
-  }
+  for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(v[i]));
+  // in pairs: what rounds in a sum of equal values in order is the same in every sub-block, and the
+  // minima's terms add it up (q5_K 600x5120, x = 0.1 everywhere: 2.2e-5 off 64 bits, in pairs 9.8e-7)
+  float p[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) p[i] = v[2 * i] + v[2 * i + 1];
+  float sum = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
   amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
   sum += __shfl_xor(sum, 1, 64);
   int e = 0;
